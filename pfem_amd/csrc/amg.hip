@@ -448,8 +448,8 @@ __device__ __forceinline__ void post_ell(const AmgView<T>& V, const BlockTask& t
     for (long long c = (long long)task.block * kWaves + (threadIdx.x >> 6); c < V.AP.nsl;
          c += (long long)task.nblocks * kWaves) {
         T y[kMaxNf];
-        if (V.APf.vals) ell_rows<NF>(V.APf, V.next_z, c, lane, y);
-        else ell_rows<NF>(V.AP, V.next_z, c, lane, y);
+        if (V.APf.vals) ell_rows<NF>(V.APf, V.next_z.get(), c, lane, y);
+        else ell_rows<NF>(V.AP, V.next_z.get(), c, lane, y);
         const long long i = c * kEllSlice + lane;
         if (i >= N) continue;
         T d[NF];

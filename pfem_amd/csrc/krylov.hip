@@ -122,7 +122,7 @@ __global__ __launch_bounds__(kBlock) void k_kry_init(const KrylovView<T>* __rest
     for (long long l = (long long)sg.lb * NPB + threadIdx.x / L; l < sg.ns; l += (long long)sg.cnt * NPB) {
         const long long i = sg.n0 + l;
         T ax[kMaxNf] = {T(0), T(0), T(0), T(0)};
-        if (!V.x_zero) node_spmv<L>(V.A, V.x, i, lane, ax);
+        if (!V.x_zero) node_spmv<L>(V.A, V.x.get(), i, lane, ax);
         if (lane < V.nf) {
             const long long row = i + (long long)lane * V.nodes;
             const T bi = V.b[row];
@@ -234,7 +234,7 @@ __device__ __forceinline__ void kry_v_nodes(const KrylovView<T>& V, const NodeMa
     for (long long l = (long long)sg.lb * NPB + threadIdx.x / L; l < sg.ns; l += (long long)sg.cnt * NPB) {
         const long long i = sg.n0 + l;
         T y[kMaxNf];
-        node_spmv<L>(A, V.ph, i, lane, y);
+        node_spmv<L>(A, V.ph.get(), i, lane, y);
         if (lane < V.nf) {
             const long long row = i + (long long)lane * V.nodes;
             const T yv = pick(y, lane);
@@ -348,7 +348,7 @@ __device__ __forceinline__ void kry_t_nodes(const KrylovView<T>& V, const NodeMa
     for (long long l = (long long)sg.lb * NPB + threadIdx.x / L; l < sg.ns; l += (long long)sg.cnt * NPB) {
         const long long i = sg.n0 + l;
         T y[kMaxNf];
-        node_spmv<L>(A, V.sh, i, lane, y);
+        node_spmv<L>(A, V.sh.get(), i, lane, y);
         if (lane < V.nf) {
             const long long row = i + (long long)lane * V.nodes;
             const T yv = pick(y, lane);
@@ -449,7 +449,7 @@ __global__ __launch_bounds__(kBlock) void k_ir_residual(const RefineView* __rest
     double part[2] = {0.0, 0.0};
     for (long long i = (long long)task.block * NPB + threadIdx.x / L; i < V.A.N; i += (long long)task.nblocks * NPB) {
         double ax[kMaxNf];
-        node_spmv<L>(V.A, V.x, i, lane, ax);
+        node_spmv<L>(V.A, V.x.get(), i, lane, ax);
         if (lane < V.A.nf) {
             const long long row = i + (long long)lane * V.A.N;
             const double bi = V.b[row];

@@ -247,7 +247,7 @@ __global__ __launch_bounds__(kBlock) void k_pspg_elem(const PspgView* __restrict
         double4* out = reinterpret_cast<double4*>(V.erec + e * kRecW);
 #pragma unroll
         for (int q = 0; q < 4; ++q) out[q] = make_double4(rec[4 * q], rec[4 * q + 1], rec[4 * q + 2], rec[4 * q + 3]);
-        reinterpret_cast<double4*>(V.esv)[e] = make_double4(sv[0], sv[1], sv[2], sv[3]);
+        reinterpret_cast<double4*>(V.esv.get())[e] = make_double4(sv[0], sv[1], sv[2], sv[3]);
     }
 }
 
@@ -460,7 +460,7 @@ __global__ __launch_bounds__(kBlock) void k_pspg_diag(const PspgView* __restrict
             add_block<D>(R, a, a, mom, blk);
             // be (MomContEquationPSPG.inl:53): F + Me/dt vPrev ; H + C tau/dt vPrev, with
             // sum_c M_ac v_c = |e| (v_a + sum_c v_c) / ((d+1)(d+2))
-            const double4 sv4 = reinterpret_cast<const double4*>(V.esv)[e];
+            const double4 sv4 = reinterpret_cast<const double4*>(V.esv.get())[e];
             const double sv[3] = {sv4.x, sv4.y, sv4.z};
             double hg = 0, cv = 0;
             double ga[D];

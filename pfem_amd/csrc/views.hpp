@@ -7,44 +7,67 @@
 
 namespace pfem {
 
+// A device-memory pointer held in a view.  The views live in memory, so the compiler cannot see
+// which address space a plain pointer loaded from one refers to and makes every access through
+// it a flat one: that goes through the LDS unit as well, takes its whole 64-bit address in
+// vector registers, and is waited for together with every other access in flight.  Held as a
+// pointer into global memory, accesses through it are global ones.  Measured
+// (same bits): steps of a 12k-node 3D column 16.65 -> 16.24 ms, of a 48k-node Delaunay mesh 66.4 ->
+// 64.1 ms, of a 20k-node 2D column 27.95 -> 27.37 ms; the compressible tile passes, which also
+// use the LDS, 537 -> 443 us.
+#if defined(__HIP_DEVICE_COMPILE__)
+#define PFEM_GLOBAL __attribute__((address_space(1)))
+#else
+#define PFEM_GLOBAL
+#endif
+template <class T>
+struct Gp {
+    PFEM_GLOBAL T* p = nullptr;
+    __host__ __device__ Gp() = default;
+    __host__ __device__ Gp(T* q) : p((PFEM_GLOBAL T*)q) {}
+    __host__ __device__ __forceinline__ T* get() const { return (T*)p; }
+    __host__ __device__ __forceinline__ operator T*() const { return (T*)p; }
+    __host__ __device__ __forceinline__ T* operator->() const { return (T*)p; }
+};
+
 // Surface-tension facets of a case (fst.hpp gathers them per node).
 struct FstView {
     int F = 0;                  // facets (0: no surface tension)
     int all_nodes = 0;          // 1: a facet acts when every node is on the free surface (WC), 0: any node
-    const int* nodes = nullptr; // [F][dim] facet nodes (Facet::m_nodesIndexes order)
-    const int* elem = nullptr;  // [F] element of each facet
-    const int* ptr = nullptr;   // [N+1] node -> entries
-    const unsigned* ent = nullptr;  // f << 2 | a, a the node's local index in the facet's element
-    const double* T = nullptr;  // Boussinesq node temperatures (null: the factor is gamma)
+    Gp<const int> nodes; // [F][dim] facet nodes (Facet::m_nodesIndexes order)
+    Gp<const int> elem;  // [F] element of each facet
+    Gp<const int> ptr;   // [N+1] node -> entries
+    Gp<const unsigned> ent;  // f << 2 | a, a the node's local index in the facet's element
+    Gp<const double> T;  // Boussinesq node temperatures (null: the factor is gamma)
     double gamma = 0, dgdT = 0, t_ref = 0;
 };
 
 // PSPG assembly + boundary conditions (MomContEquationPSPG.inl:7-235).
 struct PspgView {
     int dim, N, E, mom_nnz;
-    const int* conn;          // [ne][E]
-    const double* pos;        // [dim][N]
-    const double* q_prev;     // [(dim+1)N]  states at the start of the time step (be, free-node rhs)
-    const double* q_iter;     // [(dim+1)N]  current Picard iterate (node states used by tau)
-    const int4* node_info;    // [N] {mom_ptr, cont_ptr, deg, flags}
-    const int* nbr_ptr;       // [N+1] node graph
-    const int* nbr_idx;       // [graph_nnz]
-    const int* pei_ptr;       // [graph_nnz+1] pair-element incidence
-    const uint32_t* pei;      // [E*ne*ne]  e << 4 | a << 2 | b, sorted by e within each pair
-    const double* dir_vals;   // [dim][N] Dirichlet velocities (read at Dirichlet nodes)
-    double* vals;             // [nnz]
-    double* b;                // [(dim+1)N]
-    float* vals32;            // [nnz] FP32 copy for the mixed-precision inner solve (may be null)
-    const int* diag_pos;      // [n]
+    Gp<const int> conn;          // [ne][E]
+    Gp<const double> pos;        // [dim][N]
+    Gp<const double> q_prev;     // [(dim+1)N]  states at the start of the time step (be, free-node rhs)
+    Gp<const double> q_iter;     // [(dim+1)N]  current Picard iterate (node states used by tau)
+    Gp<const int4> node_info;    // [N] {mom_ptr, cont_ptr, deg, flags}
+    Gp<const int> nbr_ptr;       // [N+1] node graph
+    Gp<const int> nbr_idx;       // [graph_nnz]
+    Gp<const int> pei_ptr;       // [graph_nnz+1] pair-element incidence
+    Gp<const uint32_t> pei;      // [E*ne*ne]  e << 4 | a << 2 | b, sorted by e within each pair
+    Gp<const double> dir_vals;   // [dim][N] Dirichlet velocities (read at Dirichlet nodes)
+    Gp<double> vals;             // [nnz]
+    Gp<double> b;                // [(dim+1)N]
+    Gp<float> vals32;            // [nnz] FP32 copy for the mixed-precision inner solve (may be null)
+    Gp<const int> diag_pos;      // [n]
     int ell_nsl, pad_ell;     // ELL copy of the values (EllMat): slices,
-    const int* ell_soff;      // slice offsets,
-    double* vals_ell;         // values written after assembly and BC (null: none)
-    float* vals32_ell;        // FP32 ELL copy for an FP32 multigrid hierarchy (null: none)
-    double* erec;             // [E][16] element records of the assembly (pspg.hip)
-    double* esv;              // [E][4] sums of the previous-step velocities over each element
+    Gp<const int> ell_soff;      // slice offsets,
+    Gp<double> vals_ell;         // values written after assembly and BC (null: none)
+    Gp<float> vals32_ell;        // FP32 ELL copy for an FP32 multigrid hierarchy (null: none)
+    Gp<double> erec;             // [E][16] element records of the assembly (pspg.hip)
+    Gp<double> esv;              // [E][4] sums of the previous-step velocities over each element
                               //        (and, with T, of the node temperatures in the 4th slot)
-    double* binv;             // [(dim+1)^2][N] inverse diagonal node blocks (block Jacobi), SoA
-    float* binv32;            // FP32 copy for the mixed-precision inner solve (may be null)
+    Gp<double> binv;             // [(dim+1)^2][N] inverse diagonal node blocks (block Jacobi), SoA
+    Gp<float> binv32;            // FP32 copy for the mixed-precision inner solve (may be null)
     long long nnz;
     double rho, mu, dt;
     double g[3];
@@ -52,7 +75,7 @@ struct PspgView {
     double tau0, mreg;         // Bingham parameters
     // Boussinesq: node temperatures (null: none) scaling the body force of F by
     // 1 - alpha (T - Tr) at each Gauss point, and H by the same factor
-    const double* T;
+    Gp<const double> T;
     double alpha, t_ref;
     FstView fst;  // surface tension (fst.F == 0: none)
 };
@@ -66,10 +89,10 @@ template <typename T>
 struct NodeMat {
     int N, nf, mom_nnz;
     int ncol;            // nodes of the column space when it differs from the rows' (0: N)
-    const int4* info;    // [N] {mom_ptr, cont_ptr, deg, flags}
-    const int* nbr_ptr;  // [N+1]
-    const int* nbr_idx;  // [graph_nnz]
-    const T* vals;       // [nnz]
+    Gp<const int4> info;    // [N] {mom_ptr, cont_ptr, deg, flags}
+    Gp<const int> nbr_ptr;  // [N+1]
+    Gp<const int> nbr_idx;  // [graph_nnz]
+    Gp<const T> vals;       // [nnz]
 };
 
 // Node-major sliced ELL copy of a case's FP64 system (rebuilt from the values after every
@@ -84,10 +107,10 @@ template <typename VT>
 struct EllMatT {
     int N, nf, nsl;       // row nodes, fields, slices
     int ncol;             // column nodes when they differ from the rows' (0: N)
-    const int* soff;      // [nsl + 1] sum of the widths of the earlier slices
-    const int* idx;       // [soff[nsl] * 64] column node of lane r at rank k: idx[(soff[c] + k) * 64 + r]
+    Gp<const int> soff;      // [nsl + 1] sum of the widths of the earlier slices
+    Gp<const int> idx;       // [soff[nsl] * 64] column node of lane r at rank k: idx[(soff[c] + k) * 64 + r]
                           // (padding ranks: the node itself or node 0, with zero values)
-    const VT* vals;       // [soff[nsl] * nf * nf * 64] value (s, t) of lane r at rank k:
+    Gp<const VT> vals;       // [soff[nsl] * nf * nf * 64] value (s, t) of lane r at rank k:
                           // vals[((soff[c] + k) * nf * nf + s * nf + t) * 64 + r]; null: no copy
 };
 using EllMat = EllMatT<double>;
@@ -127,23 +150,23 @@ struct KrylovView {
     int amg;        // 1: ph and sh come from the multigrid V-cycle (K_p / K_s leave them)
     NodeMat<T> A;
     EllMatT<T> E;   // the ELL copy of A in type T used by K_v / K_t (vals null: node-block A)
-    const T* binv;  // [nf*nf][nodes] inverse of each node's diagonal (nf x nf) block, SoA
-    const T* b;
-    T* x;
-    T* r;
-    T* rh;
-    T* p;
-    T* v;
-    T* s;
-    T* t;
-    T* ph;
-    T* sh;
-    double* partials;    // [kMaxCaseBlocks * kPartStride]
-    unsigned* counters;  // [8]
-    KScal* sc;
+    Gp<const T> binv;  // [nf*nf][nodes] inverse of each node's diagonal (nf x nf) block, SoA
+    Gp<const T> b;
+    Gp<T> x;
+    Gp<T> r;
+    Gp<T> rh;
+    Gp<T> p;
+    Gp<T> v;
+    Gp<T> s;
+    Gp<T> t;
+    Gp<T> ph;
+    Gp<T> sh;
+    Gp<double> partials;    // [kMaxCaseBlocks * kPartStride]
+    Gp<unsigned> counters;  // [8]
+    Gp<KScal> sc;
     // FP64 multigrid: K_p / K_s also write the V-cycle's level-0 pre-smoothing w = om B^-1 p
     // (or s) from the vector they hold (null: the V-cycle's own pre-smoothing launch does it)
-    double* mg_w0;
+    Gp<double> mg_w0;
     double mg_om;
 };
 
@@ -162,53 +185,53 @@ struct AmgView {
     NodeMat<T> A;          // this level's matrix (level 0: the system or its FP32 copy)
     EllMatT<T> E0;         // level 0: the system's ELL copy in type T (vals null: none)
     EllMatT<float> E0f;    // level 0 of an FP64 hierarchy: FP32 values read by the residual (vals null: none)
-    const T* binv;         // block-Jacobi inverse, SoA [(nf*nf)][N]
+    Gp<const T> binv;         // block-Jacobi inverse, SoA [(nf*nf)][N]
     int level;
     int lanes;             // SpMV lanes per node on this level
     int mask;              // level 0: transfers and Galerkin sums use full rows only
-    const uint8_t* flags;  // level 0: the nodes' flags (the masks read them; 1 byte per node)
+    Gp<const uint8_t> flags;  // level 0: the nodes' flags (the masks read them; 1 byte per node)
     int nc;                // coarsest level: unknowns of the dense inverse
     double omega;          // block-Jacobi damping of the smoother
     double alpha;          // scaling of the coarse-grid correction (over-correction of the
                            // piecewise-constant prolongation)
-    const int* done_flag;  // the case's BiCGSTAB done flag (finished solves skip the cycle)
-    const double* r0[2];   // level 0 inputs (p, s of the FP64 BiCGSTAB)
-    double* out0[2];       // level 0 outputs (ph, sh)
-    T* r;                  // level >= 1 input
-    T* w;                  // smoothed iterate
-    T* t;                  // residual
-    T* z;                  // level >= 1 output
+    Gp<const int> done_flag;  // the case's BiCGSTAB done flag (finished solves skip the cycle)
+    Gp<const double> r0[2];   // level 0 inputs (p, s of the FP64 BiCGSTAB)
+    Gp<double> out0[2];       // level 0 outputs (ph, sh)
+    Gp<T> r;                  // level >= 1 input
+    Gp<T> w;                  // smoothed iterate
+    Gp<T> t;                  // residual
+    Gp<T> z;                  // level >= 1 output
     // transfer to the next coarser level
     int next_N;
     int pad0;
-    const int* agg_ptr;    // members (nodes of this level) of each next-level aggregate
-    const int* agg_nodes;
-    const int* fine_agg;   // next-level aggregate of each node of this level (-1: none)
-    T* next_r;
-    const T* next_z;
+    Gp<const int> agg_ptr;    // members (nodes of this level) of each next-level aggregate
+    Gp<const int> agg_nodes;
+    Gp<const int> fine_agg;   // next-level aggregate of each node of this level (-1: none)
+    Gp<T> next_r;
+    Gp<const T> next_z;
     // A P in the sliced ELL layout: this level's rows, the next coarser level's columns; the
     // entry block (i, J) sums the blocks (i, j) of i's neighbours j in aggregate J (level 0:
     // over full rows (j, t) only; zero in rows (i, s) that hold only their diagonal)
     EllMatT<T> AP;
     int ap_lanes;          // lanes per node of the set-up kernel
     int pad1;
-    const int* ap_ptr;     // [N + 1] AP entries of each node (ranks 0 .. degree-1 of its ELL row)
-    const int* ap_gptr;    // [AP entries + 1] gather list of each AP entry
-    const int* ap_gsrc;    // rank k in i's neighbour list of each gathered block
-    T* ap_out;             // AP values (written at set-up, padding ranks included)
+    Gp<const int> ap_ptr;     // [N + 1] AP entries of each node (ranks 0 .. degree-1 of its ELL row)
+    Gp<const int> ap_gptr;    // [AP entries + 1] gather list of each AP entry
+    Gp<const int> ap_gsrc;    // rank k in i's neighbour list of each gathered block
+    Gp<T> ap_out;             // AP values (written at set-up, padding ranks included)
     EllMatT<float> APf;    // level 0 of an FP64 hierarchy: AP held in FP32 instead (vals null: none)
-    float* ap_out32;       // its values (written at set-up in place of ap_out)
+    Gp<float> ap_out32;       // its values (written at set-up in place of ap_out)
     // setup of this level (>= 1) from the finer level: entry block (I, J) is the sum of the
     // finer level's A P blocks (i, J) over the members i of aggregate I
     EllMatT<T> FAP;        // the finer level's A P
     EllMatT<float> FAPf;   // ... or its FP32 copy (level 1 of an FP64 hierarchy whose level 0
                            // holds A P in FP32; vals null: none)
-    const int* gal_ptr;    // [entries + 1] gather list of each entry of this level
-    const int2* gal_src;   // {finer node i, rank m of J in i's A P row}
-    const int* self_rank;
-    T* vals_out;
-    T* binv_out;
-    double* dense;  // coarsest: [nc * nc] inverse, row major over unknowns I + s N (FP64 in
+    Gp<const int> gal_ptr;    // [entries + 1] gather list of each entry of this level
+    Gp<const int2> gal_src;   // {finer node i, rank m of J in i's A P row}
+    Gp<const int> self_rank;
+    Gp<T> vals_out;
+    Gp<T> binv_out;
+    Gp<double> dense;  // coarsest: [nc * nc] inverse, row major over unknowns I + s N (FP64 in
                     // either type: the coarse operators are the worst conditioned)
 };
 
@@ -216,14 +239,14 @@ struct AmgView {
 struct RefineView {
     int n, pad;
     NodeMat<double> A;   // FP64 system
-    const double* b;
-    double* x;           // FP64 solution
-    double* r;           // FP64 residual
-    float* r32;          // inner right-hand side
-    const float* d32;    // inner correction
-    double* partials;
-    unsigned* counters;
-    double* out;         // [4] {||r||^2, ||b||^2, ...}
+    Gp<const double> b;
+    Gp<double> x;           // FP64 solution
+    Gp<double> r;           // FP64 residual
+    Gp<float> r32;          // inner right-hand side
+    Gp<const float> d32;    // inner correction
+    Gp<double> partials;
+    Gp<unsigned> counters;
+    Gp<double> out;         // [4] {||r||^2, ||b||^2, ...}
 };
 
 // Lanes per node of the weakly compressible node-gather passes (2D, 3D): a P1 node has
@@ -236,26 +259,26 @@ constexpr int kWcLanes[2] = {8, 8};
 template <typename S>
 struct WcView {
     int dim, N, E, pad;
-    const int* conn;          // [ne][E]
-    const uint8_t* flags;     // [N] with NODE_FREE derived
-    const int* elem_ptr;      // [N+1] node-element incidence (Pattern::elem_ptr / elem_list /
-    const uint32_t* elem_list;  //       elem_nodes)
-    const int4* elem_nodes;
-    double* pos;              // [dim][N]
-    S* v;                     // [dim][N]
-    S* a;                     // [dim][N]
-    S* p;                     // [N]
-    S* rho;                   // [N]
-    const double* dir_vals;   // [dim][N]
-    double* m_cont;           // [N] lumped continuity mass of each node
-    double* f_cont;           // [N] continuity rhs
-    double* m_mom;            // [N] lumped momentum mass (same for every component)
-    double* f_mom;            // [dim][N] momentum force
-    double* hmin;             // [N] smallest he of each node's elements (CFL after the step)
-    double* rec;              // [N][8] node records {x, y, z, p, vx, vy, vz, rho} (FP64; 2D: z = vz = 0),
+    Gp<const int> conn;          // [ne][E]
+    Gp<const uint8_t> flags;     // [N] with NODE_FREE derived
+    Gp<const int> elem_ptr;      // [N+1] node-element incidence (Pattern::elem_ptr / elem_list /
+    Gp<const uint32_t> elem_list;  //       elem_nodes)
+    Gp<const int4> elem_nodes;
+    Gp<double> pos;              // [dim][N]
+    Gp<S> v;                     // [dim][N]
+    Gp<S> a;                     // [dim][N]
+    Gp<S> p;                     // [N]
+    Gp<S> rho;                   // [N]
+    Gp<const double> dir_vals;   // [dim][N]
+    Gp<double> m_cont;           // [N] lumped continuity mass of each node
+    Gp<double> f_cont;           // [N] continuity rhs
+    Gp<double> m_mom;            // [N] lumped momentum mass (same for every component)
+    Gp<double> f_mom;            // [dim][N] momentum force
+    Gp<double> hmin;             // [N] smallest he of each node's elements (CFL after the step)
+    Gp<double> rec;              // [N][8] node records {x, y, z, p, vx, vy, vz, rho} (FP64; 2D: z = vz = 0),
                               // written by the node passes, read by the element gathers
-    double* erec;             // [E][4] continuity element records {|e|, div v, sum P, 0} (FP64)
-    unsigned long long* dt2;  // CFL min accumulator (bits of a positive double)
+    Gp<double> erec;             // [E][4] continuity element records {|e|, div v, sum P, 0} (FP64)
+    Gp<unsigned long long> dt2;  // CFL min accumulator (bits of a positive double)
     double mu, K0, K0p, rho_star;
     double g[3];
     double dt;   // time step of the current launch
@@ -268,17 +291,17 @@ struct WcView {
 struct PicardView {
     int dim, N, n, res_kind;  // res_kind: 0 U, 1 U_P, 2 Ax_f
     double dt;
-    const uint8_t* flags;
-    double* pos;
-    double* pos_save;
-    double* q_prev;  // state at the start of the step (committed when the loop converges)
-    double* x;       // Picard iterate q
-    double* x_prev;  // previous iterate (U / U_P residuals)
+    Gp<const uint8_t> flags;
+    Gp<double> pos;
+    Gp<double> pos_save;
+    Gp<double> q_prev;  // state at the start of the step (committed when the loop converges)
+    Gp<double> x;       // Picard iterate q
+    Gp<double> x_prev;  // previous iterate (U / U_P residuals)
     NodeMat<double> A;
-    const double* b;
-    double* partials;
-    unsigned* counters;
-    double* out;  // [4]
+    Gp<const double> b;
+    Gp<double> partials;
+    Gp<unsigned> counters;
+    Gp<double> out;  // [4]
 };
 
 // Bookkeeping copies of the Picard step, one bit per copy (BlockTask::pad of the copy table).

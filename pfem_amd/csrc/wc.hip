@@ -112,7 +112,7 @@ __global__ __launch_bounds__(kBlock) void k_wc_half(const WcView<S>* __restrict_
             xr[k] = x;
             vr[k] = (double)vs;
         }
-        double4* R = reinterpret_cast<double4*>(V.rec) + 2 * (long long)i;
+        double4* R = reinterpret_cast<double4*>(V.rec.get()) + 2 * (long long)i;
         R[0] = make_double4(xr[0], xr[1], xr[2], (double)V.p[i]);
         R[1] = make_double4(vr[0], vr[1], vr[2], (double)V.rho[i]);
     }
@@ -160,7 +160,7 @@ __global__ __launch_bounds__(kBlock) void k_wc_cont_elem(const WcView<S>* __rest
             for (int k = 0; k < D; ++k) divv += G.gN[k][a] * vel[k][a];
         }
         // he for the CFL time step after this step (positions do not move again in it)
-        reinterpret_cast<double4*>(V.erec)[e] = make_double4(G.vol, divv, psum, elem_he<D>(x, G.vol));
+        reinterpret_cast<double4*>(V.erec.get())[e] = make_double4(G.vol, divv, psum, elem_he<D>(x, G.vol));
     }
 }
 
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(kBlock) void k_wc_cont_gather(const WcView<S>* __re
     const double dt = V.dt;
     const double c2 = 1.0 / (double)((D + 1) * (D + 2));
     const int lane = threadIdx.x % L;
-    const double4* __restrict__ erec = reinterpret_cast<const double4*>(V.erec);
+    const double4* __restrict__ erec = reinterpret_cast<const double4*>(V.erec.get());
     for (long long i = (long long)task.block * NPB + threadIdx.x / L; i < N; i += (long long)task.nblocks * NPB) {
         const int q1 = V.elem_ptr[i + 1];
         const double Pm = (double)V.p[i];
