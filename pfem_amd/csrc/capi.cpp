@@ -335,10 +335,10 @@ size_t wc_state_size(pfem_case* c) { return c->d.wc_state == PFEM_STATE_FP32 ? s
 
 size_t persistent_bytes(pfem_case* c) {
     size_t b = 0;
-    for (DevBuf* p : {&c->pos, &c->dir_vals, &c->q_prev, &c->partials, &c->counters, &c->wstate, &c->wacc, &c->wrec, &c->werec,
+    for (DevBuf* p : {&c->pos, &c->dir_vals, &c->q_prev, &c->partials, &c->counters, &c->wstate, &c->wacc,
                       &c->pat.conn, &c->pat.flags, &c->pat.nbr_ptr, &c->pat.nbr_idx, &c->pat.node_info,
                       &c->pat.row_ptr, &c->pat.diag_pos, &c->pat.pei_ptr, &c->pat.pei, &c->pat.elem_ptr,
-                      &c->pat.elem_list, &c->pat.elem_nodes, &c->pat.ell_soff, &c->pat.ell_idx})
+                      &c->pat.elem_list, &c->pat.tile_own, &c->pat.tile_nodes, &c->pat.visit, &c->pat.ell_soff, &c->pat.ell_idx})
         b += p->bytes;
     auto& H = c->heat;
     for (DevBuf* p : {&H.row_ptr, &H.col, &H.diag_pos, &H.vals, &H.b, &H.erec, &H.facets, &H.fout, &H.fkind, &H.qgp,
@@ -699,10 +699,8 @@ int pfem_case_set_mesh(pfem_case* c, int32_t N, int32_t E, const int32_t* conn, 
             const size_t ss = wc_state_size(c);
             c->wstate.reserve(ss * (size_t)(2 * dim + 2) * N);
             PFEM_HIP(hipMemsetAsync(c->wstate.p, 0, ss * (size_t)(2 * dim + 2) * N, c->stream));
-            c->wacc.reserve(sizeof(double) * (size_t)(4 + dim) * N);
-            c->wrec.reserve(sizeof(double) * 8 * (size_t)N);
-            c->werec.reserve(sizeof(double) * 4 * (size_t)E);
-            PFEM_HIP(hipMemsetAsync(c->wrec.p, 0, sizeof(double) * 8 * (size_t)N, c->stream));
+            // momentum mass and force, smallest he (FP64); half-step velocity, old pressure (state type)
+            c->wacc.reserve((sizeof(double) * (size_t)(2 + dim) + ss * (size_t)(dim + 1)) * N);
         }
         PFEM_HIP(hipStreamSynchronize(c->stream));
         c->setup_s[3] = std::chrono::duration<double>(std::chrono::steady_clock::now() - t_start).count();

@@ -78,14 +78,14 @@ __device__ __forceinline__ double dpp_mov(double v) {
     return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 
-// Sum over each aligned group of L lanes (L = 4, 8 or 16), returned in every lane of the
+// Sum over each aligned group of L lanes (L = 2, 4, 8 or 16), returned in every lane of the
 // group.  The partner sums are symmetric, so all lanes of a group hold the same bits.  Every
 // lane of a group must be active (groups never straddle a DPP row, so other groups may not be).
 template <int L, typename T>
 __device__ __forceinline__ T group_sum(T v) {
-    static_assert(L == 4 || L == 8 || L == 16, "group width");
+    static_assert(L == 2 || L == 4 || L == 8 || L == 16, "group width");
     v += dpp_mov<0xB1>(v);
-    v += dpp_mov<0x4E>(v);
+    if (L >= 4) v += dpp_mov<0x4E>(v);
     if (L >= 8) v += dpp_mov<0x141>(v);
     if (L >= 16) v += dpp_mov<0x140>(v);
     return v;
@@ -95,9 +95,9 @@ __device__ __forceinline__ T group_sum(T v) {
 // rules as group_sum).
 template <int L>
 __device__ __forceinline__ double group_min(double v) {
-    static_assert(L == 4 || L == 8 || L == 16, "group width");
+    static_assert(L == 2 || L == 4 || L == 8 || L == 16, "group width");
     v = fmin(v, dpp_mov<0xB1>(v));
-    v = fmin(v, dpp_mov<0x4E>(v));
+    if (L >= 4) v = fmin(v, dpp_mov<0x4E>(v));
     if (L >= 8) v = fmin(v, dpp_mov<0x141>(v));
     if (L >= 16) v = fmin(v, dpp_mov<0x140>(v));
     return v;

@@ -52,9 +52,9 @@ int res_kind_of(const Req* r) { return r->res_kind >= 0 ? r->res_kind : r->c->d.
 enum Tab : int {
     T_COPY, T_UPD, T_ASM2, T_ASM3, T_BC, T_RESU, T_IRU,
     T_RES, T_IRR = T_RES + 3, T_K64 = T_IRR + 3, T_K32 = T_K64 + 3, T_F64 = T_K32 + 3, T_F32 = T_F64 + 3,
-    T_WCN = T_F32 + 3, T_WCE2 = T_WCN + 2, T_WCE3 = T_WCE2 + 2, T_CFE2 = T_WCE3 + 2, T_CFE3 = T_CFE2 + 2,
-    T_WEL2 = T_CFE3 + 2, T_WEL3 = T_WEL2 + 2,  // WC continuity element pass (one lane per element)
-    T_AMG = T_WEL3 + 2,  // multigrid tables: FP64 hierarchies, then FP32 ones (A_N each)
+    T_WCN = T_F32 + 3, T_WCT2 = T_WCN + 2, T_WCT3 = T_WCT2 + 2, T_CFE2 = T_WCT3 + 2, T_CFE3 = T_CFE2 + 2,
+    T_WCF = T_CFE3 + 2,  // WC node pass of the cases with surface-tension facets
+    T_AMG = T_WCF + 2,  // multigrid tables: FP64 hierarchies, then FP32 ones (A_N each)
 };
 
 // Multigrid tables of one hierarchy type, relative to T_AMG + type * A_N: setup per level
@@ -650,7 +650,10 @@ void Engine::Impl::load_views(Req* r) {
             V.flags = c->pat.flags.as<uint8_t>();
             V.elem_ptr = c->pat.elem_ptr.as<int>();
             V.elem_list = c->pat.elem_list.as<uint32_t>();
-            V.elem_nodes = c->pat.elem_nodes.as<int4>();
+            V.ntiles = c->pat.ntiles;
+            V.tile_own = c->pat.tile_own.as<int>();
+            V.tile_nodes = c->pat.tile_nodes.as<int>();
+            V.visit = c->pat.visit.as<uint32_t>();
             V.pos = c->pos.as<double>();
             // layout of pfem_case_set_state: v (dim x N), p (N), rho (N), a (dim x N)
             V.v = base;
@@ -659,13 +662,11 @@ void Engine::Impl::load_views(Req* r) {
             V.a = base + (size_t)(dim + 2) * N;
             V.dir_vals = c->dir_vals.as<double>();
             double* acc = c->wacc.as<double>();
-            V.m_cont = acc;
-            V.f_cont = acc + N;
-            V.m_mom = acc + 2 * (size_t)N;
-            V.f_mom = acc + 3 * (size_t)N;
-            V.hmin = acc + (3 + (size_t)dim) * N;
-            V.rec = c->wrec.as<double>();
-            V.erec = c->werec.as<double>();
+            V.m_mom = acc;
+            V.f_mom = acc + N;
+            V.hmin = acc + (1 + (size_t)dim) * N;
+            V.vh = reinterpret_cast<S*>(acc + (2 + (size_t)dim) * N);
+            V.p_old = V.vh + (size_t)dim * N;
             V.dt2 = &ds->dt2;
             V.mu = c->d.mu;
             V.K0 = c->d.K0;
@@ -1036,6 +1037,7 @@ void Engine::tick(std::vector<Req*>& done) {
 
     // ---- work tables ------------------------------------------------------------------
     std::vector<BlockTask> tab[T_NTAB];
+    int wc_cap[2][2] = {{0, 0}, {0, 0}};  // most nodes a WC tile stages, by state type and dimension
     for (Req* r : inflight_) {
         pfem_case* c = r->c;
         const int sl = r->slot;
@@ -1088,12 +1090,12 @@ void Engine::tick(std::vector<Req*>& done) {
         }
         const int wi = c->d.wc_state == PFEM_STATE_FP32 ? 1 : 0;
         if (op & OP_WC) {
-            // node passes: at most kMaxCaseBlocks workgroups, each folding its CFL minimum
-            // into the slot with one atomic
             append(tab[T_WCN + wi], sl, c->N, kMaxCaseBlocks);
-            // node gathers over the incident elements: kWcLanes lanes per node
-            append(tab[(c->dim == 2 ? T_WCE2 : T_WCE3) + wi], sl, (long long)c->N * kWcLanes[c->dim - 2], kElemCap);
-            append(tab[(c->dim == 2 ? T_WEL2 : T_WEL3) + wi], sl, c->E, kElemCap);
+            // each workgroup of the last pass folds its CFL minimum into the slot with one atomic
+            append(tab[(c->dim == 2 ? T_WCT2 : T_WCT3) + wi], sl, (long long)c->pat.ntiles * kBlock, 2 * kMaxCaseBlocks);
+            if (fst_view(c, true).F > 0) append(tab[T_WCF + wi], sl, c->N, kMaxCaseBlocks);
+            int& cap = wc_cap[wi][c->dim - 2];
+            cap = std::max(cap, c->pat.tile_max);
         }
         // the step's own kernels give the CFL minimum after it; the CFL pass runs on its own
         // only without a step
@@ -1271,12 +1273,13 @@ void Engine::tick(std::vector<Req*>& done) {
     if (nrun) I.par = (I.par + chunk) & 1;
     const WcView<double>* vw64 = I.d_wc64.as<WcView<double>>();
     const WcView<float>* vw32 = I.d_wc32.as<WcView<float>>();
-    if (NT(T_WCN + 0))
-        launch_wc_step<double>(vw64, T(T_WCN), NT(T_WCN), T(T_WCE2), NT(T_WCE2), T(T_WCE3), NT(T_WCE3), T(T_WEL2),
-                               NT(T_WEL2), T(T_WEL3), NT(T_WEL3), s);
-    if (NT(T_WCN + 1))
-        launch_wc_step<float>(vw32, T(T_WCN + 1), NT(T_WCN + 1), T(T_WCE2 + 1), NT(T_WCE2 + 1), T(T_WCE3 + 1),
-                              NT(T_WCE3 + 1), T(T_WEL2 + 1), NT(T_WEL2 + 1), T(T_WEL3 + 1), NT(T_WEL3 + 1), s);
+    auto wc_step = [&](auto* vw, int wi) {
+        const BlockTask* const tiles[2] = {T(T_WCT2 + wi), T(T_WCT3 + wi)};
+        const int n[2] = {NT(T_WCT2 + wi), NT(T_WCT3 + wi)};
+        if (NT(T_WCN + wi)) launch_wc_step(vw, T(T_WCN + wi), NT(T_WCN + wi), tiles, n, wc_cap[wi], T(T_WCF + wi), NT(T_WCF + wi), s);
+    };
+    wc_step(vw64, 0);
+    wc_step(vw32, 1);
     if (NT(T_CFE2) + NT(T_CFE3)) launch_wc_cfl<double>(vw64, T(T_CFE2), NT(T_CFE2), T(T_CFE3), NT(T_CFE3), s);
     if (NT(T_CFE2 + 1) + NT(T_CFE3 + 1))
         launch_wc_cfl<float>(vw32, T(T_CFE2 + 1), NT(T_CFE2 + 1), T(T_CFE3 + 1), NT(T_CFE3 + 1), s);

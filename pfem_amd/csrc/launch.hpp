@@ -49,12 +49,12 @@ void launch_update_pos(const PicardView* v, const BlockTask* t, int nt, hipStrea
 void launch_res_axf(int lanes, const PicardView* v, const BlockTask* t, int nt, hipStream_t s);
 void launch_res_u(const PicardView* v, const BlockTask* t, int nt, hipStream_t s);
 
-// node_tasks: one lane per node; gather2 / gather3: kWcLanes lanes per node of 2D / 3D cases;
-// elem2 / elem3: one lane per element of 2D / 3D cases
+// node: one lane per node; tiles[d - 2]: one workgroup per kWcTile nodes of d-dimensional cases,
+// whose tiles stage at most cap[d - 2] nodes; fst: one lane per node of the cases with
+// surface-tension facets
 template <typename S>
-void launch_wc_step(const WcView<S>* v, const BlockTask* node_tasks, int n_node_tasks, const BlockTask* gather2,
-                    int n_gather2, const BlockTask* gather3, int n_gather3, const BlockTask* elem2, int n_elem2,
-                    const BlockTask* elem3, int n_elem3, hipStream_t s);
+void launch_wc_step(const WcView<S>* v, const BlockTask* node, int n_node, const BlockTask* const (&tiles)[2],
+                    const int (&n_tiles)[2], const int (&cap)[2], const BlockTask* fst, int n_fst, hipStream_t s);
 template <typename S>
 void launch_wc_cfl(const WcView<S>* v, const BlockTask* elem2, int n_elem2, const BlockTask* elem3, int n_elem3,
                    hipStream_t s);

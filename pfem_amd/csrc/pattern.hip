@@ -10,6 +10,7 @@
 
 #include "common.hpp"
 #include "pattern.hpp"
+#include "views.hpp"
 
 namespace pfem {
 namespace {
@@ -245,17 +246,94 @@ __global__ void k_elem_fill(int E, int ne, const int* __restrict__ soa, const in
         }
 }
 
-// Nodes of the element of each node-element incidence entry (padded with -1 in 2D).
-__global__ void k_elem_nodes(long long total, int E, int ne, const int* __restrict__ soa,
-                             const uint32_t* __restrict__ list, int4* __restrict__ nodes) {
-    for (long long q = blockIdx.x * (long long)blockDim.x + threadIdx.x; q < total; q += (long long)gridDim.x * blockDim.x) {
-        const long long e = list[q] >> 2;
-        int4 v;
-        v.x = soa[e];
-        v.y = soa[(long long)E + e];
-        v.z = soa[2LL * E + e];
-        v.w = ne > 3 ? soa[3LL * E + e] : -1;
-        nodes[q] = v;
+// One workgroup per tile of T nodes: the tile's nodes and the other nodes of their elements
+// (at most kWcTileCap, the tile's own first) are collected in an LDS hash set, sorted and
+// listed, and every incidence entry of the tile's nodes gets the slots of its other nodes.
+template <int NE>
+__global__ __launch_bounds__(kBlock) void k_wc_tiles(int N, int E, int ntiles, const int* __restrict__ elem_ptr,
+                                                     const uint32_t* __restrict__ elem_list,
+                                                     const int* __restrict__ soa, int* __restrict__ own,
+                                                     int* __restrict__ nodes, uint32_t* __restrict__ visit,
+                                                     int* __restrict__ most) {
+    constexpr int D = NE - 1, T = kWcTile[D - 2], H = 2048, P = 1024;
+    static_assert(kWcTileCap + kBlock < H && kWcTileCap < P, "hash set and sort sizes");
+    __shared__ int table[H];
+    __shared__ int list[P];
+    __shared__ int cnt;
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        for (int k = threadIdx.x; k < H; k += kBlock) table[k] = -1;
+        for (int k = threadIdx.x; k < P; k += kBlock) list[k] = 0x7fffffff;
+        if (threadIdx.x == 0) cnt = 0;
+        __syncthreads();
+        const int i0 = tile * T, i1 = min(N, i0 + T);
+        auto insert = [&](int j) {
+            // a full list takes no more: at most one late node per thread enters the table after
+            // that, so a free slot always remains and the probe ends
+            if (__hip_atomic_load(&cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >= kWcTileCap) return;
+            unsigned h = ((unsigned)j * 2654435761u) >> 21;
+            for (;;) {
+                const int old = atomicCAS(&table[h], -1, j);
+                if (old == j) return;
+                if (old == -1) {
+                    const int at = atomicAdd(&cnt, 1);
+                    if (at < kWcTileCap) list[at] = j;
+                    return;
+                }
+                h = (h + 1) & (H - 1);
+            }
+        };
+        for (int i = i0 + threadIdx.x; i < i1; i += kBlock) insert(i);
+        __syncthreads();
+        const int q0 = elem_ptr[i0], q1 = elem_ptr[i1];
+        for (int q = q0 + threadIdx.x; q < q1; q += kBlock) {
+            const long long e = elem_list[q] >> 2;
+#pragma unroll
+            for (int a = 0; a < NE; ++a) insert(soa[(long long)a * E + e]);
+        }
+        __syncthreads();
+        const int n = min(cnt, kWcTileCap);
+        for (int k = 2; k <= P; k <<= 1)  // bitonic sort (unused places hold the largest int)
+            for (int j = k >> 1; j > 0; j >>= 1) {
+                for (int x = threadIdx.x; x < P; x += kBlock) {
+                    const int y = x ^ j;
+                    if (y > x) {
+                        const int u = list[x], v = list[y];
+                        if ((u > v) == ((x & k) == 0)) {
+                            list[x] = v;
+                            list[y] = u;
+                        }
+                    }
+                }
+                __syncthreads();
+            }
+        auto slot = [&](int j) {  // first place not below j
+            int lo = 0, hi = n;
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                if (list[mid] < j) lo = mid + 1;
+                else hi = mid;
+            }
+            return lo;
+        };
+        for (int k = threadIdx.x; k < kWcTileCap; k += kBlock) nodes[(long long)tile * kWcTileCap + k] = k < n ? list[k] : -1;
+        if (threadIdx.x == 0) {
+            own[tile] = slot(i0);
+            atomicMax(most, n);
+        }
+        for (int q = q0 + threadIdx.x; q < q1; q += kBlock) {
+            const uint32_t en = elem_list[q];
+            const long long e = en >> 2;
+            uint32_t w = 0;
+#pragma unroll
+            for (int m = 1; m < NE; ++m) {
+                const int j = soa[(long long)wc_other<D>((int)(en & 3u), m) * E + e];
+                const int k = slot(j);
+                if (k >= n || list[k] != j) w = kWcFar;
+                if (w != kWcFar) w |= (uint32_t)k << (10 * (m - 1));
+            }
+            visit[q] = w;
+        }
+        __syncthreads();
     }
 }
 
@@ -322,10 +400,22 @@ void build_mesh_basic(int dim, int N, int E, const int* conn_aos, const uint8_t*
     k_pei_sort<<<grid_for(N, kBlock, 65536), kBlock, 0, stream>>>(N, pat.elem_ptr.as<int>(),
                                                                   pat.elem_list.as<uint32_t>());
     const long long total = (long long)E * ne;
-    pat.elem_nodes.reserve(sizeof(int4) * (size_t)total);
-    k_elem_nodes<<<grid_for(total, kBlock, 65536), kBlock, 0, stream>>>(total, E, ne, pat.conn.as<int>(),
-                                                                        pat.elem_list.as<uint32_t>(),
-                                                                        pat.elem_nodes.as<int4>());
+    pat.ntiles = (N + kWcTile[dim - 2] - 1) / kWcTile[dim - 2];
+    pat.tile_own.reserve(sizeof(int) * (size_t)pat.ntiles);
+    pat.tile_nodes.reserve(sizeof(int) * (size_t)pat.ntiles * kWcTileCap);
+    pat.visit.reserve(sizeof(uint32_t) * (size_t)total);
+    PFEM_HIP(hipMemsetAsync(err.p, 0, sizeof(int), stream));
+    const int gb = grid_for(pat.ntiles, 1, 65536);
+    if (dim == 2)
+        k_wc_tiles<3><<<gb, kBlock, 0, stream>>>(N, E, pat.ntiles, pat.elem_ptr.as<int>(), pat.elem_list.as<uint32_t>(),
+                                                 pat.conn.as<int>(), pat.tile_own.as<int>(), pat.tile_nodes.as<int>(),
+                                                 pat.visit.as<uint32_t>(), err.as<int>());
+    else
+        k_wc_tiles<4><<<gb, kBlock, 0, stream>>>(N, E, pat.ntiles, pat.elem_ptr.as<int>(), pat.elem_list.as<uint32_t>(),
+                                                 pat.conn.as<int>(), pat.tile_own.as<int>(), pat.tile_nodes.as<int>(),
+                                                 pat.visit.as<uint32_t>(), err.as<int>());
+    PFEM_HIP(hipGetLastError());
+    PFEM_HIP(hipMemcpyAsync(&pat.tile_max, err.p, sizeof(int), hipMemcpyDeviceToHost, stream));
     PFEM_HIP(hipStreamSynchronize(stream));
 }
 

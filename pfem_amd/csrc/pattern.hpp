@@ -40,8 +40,12 @@ struct Pattern {
     // elem_ptr[i] .. elem_ptr[i+1] hold e << 2 | a with conn[e][a] = i, sorted by element
     DevBuf elem_ptr;   // int  [N + 1]
     DevBuf elem_list;  // u32  [E * ne]
-    DevBuf elem_nodes; // int4 [E * ne] the element's nodes (local order) of each entry, so that
-                       //      a gather over a node's elements needs no connectivity lookup
+    // tiles of the weakly compressible passes (kWcTile nodes each; views.hpp)
+    int ntiles = 0, tile_max = 0;  // tiles, most nodes staged by one
+    DevBuf tile_own;   // int  [ntiles] slot of the tile's first node
+    DevBuf tile_nodes; // int  [ntiles][kWcTileCap] staged nodes, ascending, then -1
+    DevBuf visit;      // u32  [E * ne] slots of the other nodes of each incidence entry (10 bits
+                       //      each, positive orientation with the entry's node first) or kWcFar
     // node-major sliced ELL structure (EllMat in views.hpp; PSPG cases)
     int ell_nsl = 0;          // slices of 64 nodes
     long long ell_ranks = 0;  // sum of the slice widths

@@ -249,11 +249,24 @@ struct RefineView {
     Gp<double> out;         // [4] {||r||^2, ||b||^2, ...}
 };
 
-// Lanes per node of the weakly compressible node-gather passes (2D, 3D): a P1 node has
-// ~6 incident triangles in 2D and ~24 tetrahedra in 3D.  On the 2.06M-node 3D tank the
-// momentum / continuity gathers take 991 / 284 us at 16 lanes, 830 / 255 at 8 and 919 / 312
-// at 4 (whole step 566, 626 and 572 steps/s).
-constexpr int kWcLanes[2] = {8, 8};
+// Tiles of the weakly compressible passes (2D, 3D): consecutive nodes per workgroup, lanes per
+// node (a P1 node has ~6 incident triangles in 2D and ~24 tetrahedra in 3D), the nodes that one
+// tile stages in LDS at most (72 bytes each in FP64) and the visit words staged beside them:
+// together with the static arrays within 64 KiB.  Tiles of a spatially ordered 3D mesh hold ~600
+// nodes, of a random order up to ~1,000; elements with a node beyond the capacity are visited
+// through memory (kWcFar), visit words past theirs are read from memory.
+constexpr int kWcTile[2] = {128, 64};
+constexpr int kWcTileLanes[2] = {2, 4};
+constexpr int kWcTileCap = 752;
+constexpr int kWcVisits[2] = {1024, 1792};
+constexpr uint32_t kWcFar = 0xffffffffu;
+
+// Local index of the m-th other node (m = 1..D) of an element seen from its local node me,
+// positively oriented with me first (3D: double transpositions, 2D: rotations).
+template <int D>
+__host__ __device__ constexpr int wc_other(int me, int m) {
+    return D == 3 ? (me ^ m) : (me + m) % 3;
+}
 
 // Weakly compressible explicit step (WCompNewton/Solver.cpp:236-276).
 template <typename S>
@@ -261,23 +274,23 @@ struct WcView {
     int dim, N, E, pad;
     Gp<const int> conn;          // [ne][E]
     Gp<const uint8_t> flags;     // [N] with NODE_FREE derived
-    Gp<const int> elem_ptr;      // [N+1] node-element incidence (Pattern::elem_ptr / elem_list /
-    Gp<const uint32_t> elem_list;  //       elem_nodes)
-    Gp<const int4> elem_nodes;
+    Gp<const int> elem_ptr;        // [N+1] node-element incidence (Pattern::elem_ptr / elem_list)
+    Gp<const uint32_t> elem_list;
+    int ntiles, pad_tiles;
+    Gp<const int> tile_own;      // [ntiles] LDS slot of the tile's first node
+    Gp<const int> tile_nodes;    // [ntiles][kWcTileCap] staged nodes, ascending, then -1
+    Gp<const uint32_t> visit;    // per incidence entry: LDS slots of the other nodes, 10 bits each, or kWcFar
     Gp<double> pos;              // [dim][N]
     Gp<S> v;                     // [dim][N]
     Gp<S> a;                     // [dim][N]
     Gp<S> p;                     // [N]
     Gp<S> rho;                   // [N]
     Gp<const double> dir_vals;   // [dim][N]
-    Gp<double> m_cont;           // [N] lumped continuity mass of each node
-    Gp<double> f_cont;           // [N] continuity rhs
-    Gp<double> m_mom;            // [N] lumped momentum mass (same for every component)
-    Gp<double> f_mom;            // [dim][N] momentum force
+    Gp<S> vh;                    // [dim][N] half-step velocity
+    Gp<S> p_old;                 // [N] pressure before the continuity pass
+    Gp<double> m_mom;            // [N] lumped momentum mass (cases with surface-tension facets)
+    Gp<double> f_mom;            // [dim][N] momentum force (same)
     Gp<double> hmin;             // [N] smallest he of each node's elements (CFL after the step)
-    Gp<double> rec;              // [N][8] node records {x, y, z, p, vx, vy, vz, rho} (FP64; 2D: z = vz = 0),
-                              // written by the node passes, read by the element gathers
-    Gp<double> erec;             // [E][4] continuity element records {|e|, div v, sum P, 0} (FP64)
     Gp<unsigned long long> dt2;  // CFL min accumulator (bits of a positive double)
     double mu, K0, K0p, rho_star;
     double g[3];
