@@ -668,7 +668,7 @@ def run_dambreak3d(ctx, steps, warmup):
         elements_per_s=mesh.n_elems / t_asm if t_asm > 0 else None,
     )
     roof = {
-        "kernel": "k_kry_v<double,16> (BiCGSTAB SpMV v = A ph over the sliced ELL copy, fused (rh, v)), "
+        "kernel": "k_kry_v<double> (BiCGSTAB SpMV v = A ph over the sliced ELL copy, fused (rh, v)), "
                   "3D dam break 262,701 nodes",
         "bound": "hbm",
         "achieved": achieved,

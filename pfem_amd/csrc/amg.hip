@@ -5,8 +5,9 @@
 // transfer.
 //
 // V-cycle on level l (input r_l, output z_l; level 0 reads p or s and writes ph or sh):
-//   w = omega B^-1 r                      (k_amg_pre at level 0, block-Jacobi pre-smoothing;
-//                                          on coarser levels done by the restriction above)
+//   w = omega B^-1 r                      (block-Jacobi pre-smoothing: at level 0 done by the
+//                                          BiCGSTAB kernel that forms r_0, on coarser levels by
+//                                          the restriction above)
 //   t = r - A w                           (k_amg_res)
 //   r_{l+1} = P^T t                       (k_amg_restrict, gather over aggregate members)
 //   z_{l+1} = V-cycle(l+1)  /  A_c^-1 r_c (k_amg_coarsest, dense inverse on the coarsest)
@@ -34,7 +35,8 @@ __device__ __forceinline__ long long row_start_of(const int4& inf, int s, int D,
     return (s < D) ? (long long)s * mom_nnz + inf.x : (long long)D * mom_nnz + inf.y;
 }
 
-// Entry q of the level's input (level 0: the FP64 Krylov vector p or s).
+// Entry q of the level's input (level 0: the FP64 Krylov vector p or s); every vector of the
+// V-cycle is node-blocked (entry i nf + s), as BiCGSTAB's are.
 template <typename T>
 __device__ __forceinline__ T in_at(const AmgView<T>& V, int which, long long q) {
     return V.level == 0 ? (T)V.r0[which][q] : V.r[q];
@@ -227,7 +229,7 @@ __global__ __launch_bounds__(kBlock) void k_amg_dense(const AmgView<T>* __restri
     const int n = V.nc, N = V.A.N, nf = V.A.nf, D = nf - 1;
     for (int e = threadIdx.x; e < n * n; e += kBlock) a[e] = 0.0;
     __syncthreads();
-    // scatter the node-block values: unknown (I, s) is I + s N
+    // scatter the node-block values: unknown (I, s) is I nf + s
     for (int I = threadIdx.x; I < N; I += kBlock) {
         const int4 inf = V.A.info[I];
         const int nb = V.A.nbr_ptr[I];
@@ -235,7 +237,7 @@ __global__ __launch_bounds__(kBlock) void k_amg_dense(const AmgView<T>* __restri
             const int J = V.A.nbr_idx[nb + k];
             for (int s = 0; s < nf; ++s) {
                 const long long rs = row_start_of(inf, s, D, V.A.mom_nnz) + k;
-                for (int t = 0; t < nf; ++t) a[(I + s * N) * n + (J + t * N)] = (double)V.A.vals[rs + (long long)t * inf.z];
+                for (int t = 0; t < nf; ++t) a[(I * nf + s) * n + (J * nf + t)] = (double)V.A.vals[rs + (long long)t * inf.z];
             }
         }
     }
@@ -298,31 +300,6 @@ __global__ __launch_bounds__(kBlock) void k_amg_dense(const AmgView<T>* __restri
 
 // ---- V-cycle -----------------------------------------------------------------------------
 
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_amg_pre(const AmgView<T>* __restrict__ views,
-                                                    const BlockTask* __restrict__ tasks, int which) {
-    const BlockTask task = tasks[blockIdx.x];
-    if (task.case_id < 0) return;
-    const AmgView<T>& V = views[task.case_id];
-    if (*V.done_flag) return;
-    const int nf = V.A.nf, N = V.A.N;
-    const T om = (T)V.omega;
-    for (long long i = (long long)task.block * kBlock + threadIdx.x; i < N; i += (long long)task.nblocks * kBlock) {
-        T x[kMaxNf];
-#pragma unroll
-        for (int t = 0; t < kMaxNf; ++t) x[t] = (t < nf) ? in_at(V, which, i + (long long)t * N) : T(0);
-#pragma unroll
-        for (int s = 0; s < kMaxNf; ++s) {
-            if (s >= nf) continue;
-            T acc = 0;
-#pragma unroll
-            for (int t = 0; t < kMaxNf; ++t)
-                if (t < nf) acc += V.binv[(long long)(s * nf + t) * N + i] * x[t];
-            V.w[i + (long long)s * N] = om * acc;
-        }
-    }
-}
-
 template <typename T, int L>
 __device__ __forceinline__ void res_body(const AmgView<T>& V, const BlockTask& task, int which) {
     constexpr int NPB = kBlock / L;
@@ -330,9 +307,9 @@ __device__ __forceinline__ void res_body(const AmgView<T>& V, const BlockTask& t
     const int N = V.A.N;
     for (long long i = (long long)task.block * NPB + threadIdx.x / L; i < N; i += (long long)task.nblocks * NPB) {
         T y[kMaxNf];
-        node_spmv<L>(V.A, (const T*)V.w, i, lane, y);
+        node_spmv<L, true>(V.A, (const T*)V.w, i, lane, y);
         if (lane < V.A.nf) {
-            const long long q = i + (long long)lane * N;
+            const long long q = i * V.A.nf + lane;
             V.t[q] = in_at(V, which, q) - pick(y, lane);
         }
     }
@@ -348,14 +325,15 @@ __device__ __forceinline__ void res_ell(const AmgView<T>& V, const BlockTask& ta
     const long long N = E.N;
     for (long long c = (long long)task.block * kWaves + (threadIdx.x >> 6); c < E.nsl;
          c += (long long)task.nblocks * kWaves) {
-        T y[kMaxNf];
-        if (V.E0f.vals) ell_rows<NF>(V.E0f, (const T*)V.w, c, lane, y);
-        else ell_rows<NF>(E, (const T*)V.w, c, lane, y);
+        T y[NF];
+        auto xat = [&](long long j, T (&xv)[NF]) { at_node<NF>((const T*)V.w, j, xv); };
+        if (V.E0f.vals) slice_part<NF>(V.E0f, c, 0, 1, xat, y);
+        else slice_part<NF>(E, c, 0, 1, xat, y);
         const long long i = c * kEllSlice + lane;
         if (i < N) {
 #pragma unroll
             for (int s = 0; s < NF; ++s) {
-                const long long q = i + (long long)s * N;
+                const long long q = i * NF + s;
                 V.t[q] = (T)V.r0[which][q] - y[s];
             }
         }
@@ -382,7 +360,7 @@ __global__ __launch_bounds__(kBlock) void k_amg_res(const AmgView<T>* __restrict
 // r_{l+1}(I, s) = sum over the members i of aggregate I of t(i, s) (level 0: full rows only);
 // kRestrictLanes lanes per aggregate share its members (aggregates hold 5-30 nodes).  When
 // level l+1 is not the coarsest, its pre-smoothing w_{l+1}(I) = omega B^-1(I) r_{l+1}(I) is
-// local to I and is applied here as well (level l+1 has no k_amg_pre launch).
+// local to I and is applied here as well.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_amg_restrict(const AmgView<T>* __restrict__ views,
                                                          const BlockTask* __restrict__ tasks) {
@@ -394,7 +372,7 @@ __global__ __launch_bounds__(kBlock) void k_amg_restrict(const AmgView<T>* __res
     const AmgView<T>& Vn = views[task.case_id + 1];  // level l+1 (views of a case are consecutive)
     const bool smooth = Vn.dense == nullptr;
     const T om = (T)Vn.omega;
-    const int nf = V.A.nf, D = nf - 1, N = V.A.N, Nc = V.next_N;
+    const int nf = V.A.nf, D = nf - 1, Nc = V.next_N;
     const int lane = threadIdx.x % L;
     for (long long I = (long long)task.block * NPB + threadIdx.x / L; I < Nc; I += (long long)task.nblocks * NPB) {
         double acc[kMaxNf] = {0.0, 0.0, 0.0, 0.0};
@@ -403,19 +381,19 @@ __global__ __launch_bounds__(kBlock) void k_amg_restrict(const AmgView<T>* __res
             const uint8_t f = V.mask ? V.flags[i] : (uint8_t)0;
 #pragma unroll
             for (int s = 0; s < kMaxNf; ++s)
-                if (s < nf && (!V.mask || row_full_flags(f, s, D))) acc[s] += (double)V.t[i + (long long)s * N];
+                if (s < nf && (!V.mask || row_full_flags(f, s, D))) acc[s] += (double)V.t[(long long)i * nf + s];
         }
 #pragma unroll
         for (int s = 0; s < kMaxNf; ++s)
             if (s < nf) acc[s] = group_sum<L>(acc[s]);
         if (lane < nf) {
-            V.next_r[I + (long long)lane * Nc] = (T)pick(acc, lane);
+            V.next_r[I * nf + lane] = (T)pick(acc, lane);
             if (smooth) {
                 T w = 0;
 #pragma unroll
                 for (int t = 0; t < kMaxNf; ++t)
                     if (t < nf) w += Vn.binv[(long long)(lane * nf + t) * Nc + I] * (T)acc[t];
-                Vn.w[I + (long long)lane * Nc] = om * w;
+                Vn.w[I * nf + lane] = om * w;
             }
         }
     }
@@ -442,19 +420,20 @@ __global__ __launch_bounds__(kBlock) void k_amg_coarsest(const AmgView<T>* __res
 // view holds it so (APf).
 template <int NF, typename T>
 __device__ __forceinline__ void post_ell(const AmgView<T>& V, const BlockTask& task, int which) {
-    const int N = V.A.N, D = NF - 1, Nc = V.next_N;
+    const int N = V.A.N, D = NF - 1;
     const T om = (T)V.omega, al = (T)V.alpha;
     const int lane = threadIdx.x & (kEllSlice - 1);
     for (long long c = (long long)task.block * kWaves + (threadIdx.x >> 6); c < V.AP.nsl;
          c += (long long)task.nblocks * kWaves) {
-        T y[kMaxNf];
-        if (V.APf.vals) ell_rows<NF>(V.APf, V.next_z.get(), c, lane, y);
-        else ell_rows<NF>(V.AP, V.next_z.get(), c, lane, y);
+        T y[NF];
+        auto xat = [&](long long j, T (&xv)[NF]) { at_node<NF>(V.next_z.get(), j, xv); };
+        if (V.APf.vals) slice_part<NF>(V.APf, c, 0, 1, xat, y);
+        else slice_part<NF>(V.AP, c, 0, 1, xat, y);
         const long long i = c * kEllSlice + lane;
         if (i >= N) continue;
         T d[NF];
 #pragma unroll
-        for (int t = 0; t < NF; ++t) d[t] = V.t[i + (long long)t * N] - al * y[t];
+        for (int t = 0; t < NF; ++t) d[t] = V.t[i * NF + t] - al * y[t];
         const int I = V.fine_agg[i];
         const uint8_t f = V.mask ? V.flags[i] : (uint8_t)0;
 #pragma unroll
@@ -462,9 +441,9 @@ __device__ __forceinline__ void post_ell(const AmgView<T>& V, const BlockTask& t
             T acc = 0;
 #pragma unroll
             for (int t = 0; t < NF; ++t) acc += V.binv[(long long)(s * NF + t) * N + i] * d[t];
-            const long long q = i + (long long)s * N;
+            const long long q = i * NF + s;
             T wq = V.w[q];
-            if (I >= 0 && (!V.mask || row_full_flags(f, s, D))) wq += al * V.next_z[I + (long long)s * Nc];
+            if (I >= 0 && (!V.mask || row_full_flags(f, s, D))) wq += al * V.next_z[(long long)I * NF + s];
             const T out = wq + om * acc;
             if (V.level == 0) V.out0[which][q] = (double)out;
             else V.z[q] = out;
@@ -497,10 +476,6 @@ void launch_amg_dense(const AmgView<T>* v, const BlockTask* t, int nt, hipStream
     k_amg_dense<T><<<nt, kBlock, 0, s>>>(v, t);
 }
 template <typename T>
-void launch_amg_pre(const AmgView<T>* v, const BlockTask* t, int nt, int which, hipStream_t s) {
-    k_amg_pre<T><<<nt, kBlock, 0, s>>>(v, t, which);
-}
-template <typename T>
 void launch_amg_res(const AmgView<T>* v, const BlockTask* t, int nt, int which, hipStream_t s) {
     k_amg_res<T><<<nt, kBlock, 0, s>>>(v, t, which);
 }
@@ -525,7 +500,6 @@ void launch_amg_post(const AmgView<T>* v, const BlockTask* t, int nt, int which,
     template void launch_amg_galerkin<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);   \
     template void launch_amg_bjac<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);       \
     template void launch_amg_dense<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);      \
-    template void launch_amg_pre<T>(const AmgView<T>*, const BlockTask*, int, int, hipStream_t);   \
     template void launch_amg_res<T>(const AmgView<T>*, const BlockTask*, int, int, hipStream_t);   \
     template void launch_amg_restrict<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);   \
     template void launch_amg_coarsest<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);   \

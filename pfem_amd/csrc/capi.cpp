@@ -1241,7 +1241,7 @@ int pfem_bench_kernels(pfem_case* c, int32_t reps, double* out10) {
         double* w = c->ws.kv64;
         for (int k = 0; k < 10; ++k) out10[k] = 0;
         {  // the BiCGSTAB SpMV kernel (v = A ph with the fused (rh, v)) as a solve launches it
-            const int nb = pfem::row_blocks(n, c->pat.ell_nsl);
+            const int nb = pfem::kry_blocks(c->pat.ell_nsl);
             std::vector<pfem::BlockTask> tasks((size_t)nb);
             for (int b = 0; b < nb; ++b) tasks[(size_t)b] = pfem::BlockTask{0, b, nb, 0};
             pfem::KrylovView<double> kv{};
@@ -1249,30 +1249,36 @@ int pfem_bench_kernels(pfem_case* c, int32_t reps, double* out10) {
             kv.nodes = c->N;
             kv.nf = c->dim + 1;
             kv.nblk = nb;
-            kv.A = node_mat<double>(c->pat, c->dim, c->ws.vals);
+            kv.amg = c->amg.levels > 1 ? 1 : 0;
+            kv.split = pfem::kry_split(c->pat.ell_nsl);
             kv.E.N = c->N;
             kv.E.nf = c->dim + 1;
             kv.E.nsl = c->pat.ell_nsl;
             kv.E.soff = c->pat.ell_soff.as<int>();
             kv.E.idx = c->pat.ell_idx.as<int>();
             kv.E.vals = c->ws.vals_ell;
+            kv.binv = c->ws.binv;
             kv.ph = c->q_prev.as<double>();
             kv.rh = w;
             kv.v = w + n;
+            kv.s = w + 2LL * n;
             kv.partials = c->partials.as<double>();
-            kv.counters = c->counters.as<unsigned>();
+            pfem::KScal sc{};  // a running solve: (r, r) = 0 is above this tolerance
+            sc.tol2 = -1.0;
+            sc.maxit = 1;
             DevBuf d_tasks, d_view, d_sc;
             d_tasks.reserve(sizeof(pfem::BlockTask) * tasks.size());
             d_view.reserve(sizeof(kv));
-            d_sc.reserve(sizeof(pfem::KScal));
-            PFEM_HIP(hipMemsetAsync(d_sc.p, 0, sizeof(pfem::KScal), c->stream));  // done = 0: the kernel runs
+            d_sc.reserve(sizeof(sc));
             kv.sc = d_sc.as<pfem::KScal>();
+            PFEM_HIP(hipMemsetAsync(c->partials.p, 0, c->partials.bytes, c->stream));
+            PFEM_HIP(hipMemcpyAsync(d_sc.p, &sc, sizeof(sc), hipMemcpyHostToDevice, c->stream));
             PFEM_HIP(hipMemcpyAsync(d_tasks.p, tasks.data(), sizeof(pfem::BlockTask) * tasks.size(),
                                     hipMemcpyHostToDevice, c->stream));
             PFEM_HIP(hipMemcpyAsync(d_view.p, &kv, sizeof(kv), hipMemcpyHostToDevice, c->stream));
             out8[0] = timed([&] {
-                pfem::launch_kry_phase<double>(1, c->lanes, d_view.as<pfem::KrylovView<double>>(),
-                                               d_tasks.as<pfem::BlockTask>(), nb, 0, c->stream, nullptr);
+                pfem::launch_kry_phase<double>(1, d_view.as<pfem::KrylovView<double>>(), d_tasks.as<pfem::BlockTask>(),
+                                               nb, 0, c->stream);
             });
         }
         if (c->d.precision == PFEM_PREC_MIXED_IR) {

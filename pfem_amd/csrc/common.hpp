@@ -103,10 +103,19 @@ __device__ __forceinline__ double group_min(double v) {
     return v;
 }
 
+// Lane l's value in every lane (l a constant).
+__device__ __forceinline__ double lane_of(double v, int l) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+
+// Sum over the wavefront, in every lane; every lane must be active.  The four 16-lane rows by
+// DPP, then the rows' sums in order through scalar registers: no LDS round trips (a
+// reduction sits at the head of every BiCGSTAB kernel).
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    v = group_sum<16>(v);
+    return ((lane_of(v, 0) + lane_of(v, 16)) + lane_of(v, 32)) + lane_of(v, 48);
 }
 
 __device__ __forceinline__ double wave_max(double v) {

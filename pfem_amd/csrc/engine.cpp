@@ -51,8 +51,8 @@ int res_kind_of(const Req* r) { return r->res_kind >= 0 ? r->res_kind : r->c->d.
 
 enum Tab : int {
     T_COPY, T_UPD, T_ASM2, T_ASM3, T_BC, T_RESU, T_IRU,
-    T_RES, T_IRR = T_RES + 3, T_K64 = T_IRR + 3, T_K32 = T_K64 + 3, T_F64 = T_K32 + 3, T_F32 = T_F64 + 3,
-    T_WCN = T_F32 + 3, T_WCT2 = T_WCN + 2, T_WCT3 = T_WCT2 + 2, T_CFE2 = T_WCT3 + 2, T_CFE3 = T_CFE2 + 2,
+    T_RES, T_IRR = T_RES + 3, T_K64 = T_IRR + 3, T_K32, T_F64, T_F32,
+    T_WCN, T_WCT2 = T_WCN + 2, T_WCT3 = T_WCT2 + 2, T_CFE2 = T_WCT3 + 2, T_CFE3 = T_CFE2 + 2,
     T_WCF = T_CFE3 + 2,  // WC node pass of the cases with surface-tension facets
     T_AMG = T_WCF + 2,  // multigrid tables: FP64 hierarchies, then FP32 ones (A_N each)
 };
@@ -133,6 +133,15 @@ int row_blocks(long long n, int nsl) {
         nb = std::max<long long>(nb, kXcd * ((waves + kWaves - 1) / kWaves));
     }
     return (int)nb;
+}
+
+// A workgroup's wavefronts share a slice while all the workgroups run at once (768: three per CU;
+// their registers allow four).  Measured per iteration, shared / one wavefront per slice: 188
+// slices (12k nodes, 3D FP64) 31 / 46 us, 16 (1k, 2D) 16 / 19, 313 (20k, 2D, multigrid's part) 25 /
+// 33, 750 (48k, 3D FP64) 76 / 75, 1,125 (72k, 3D FP32) 67 / 54, 4,110 (263k, 3D FP64) 260 / 228.
+bool kry_split(int nsl) { return nsl <= 768; }
+int kry_blocks(int nsl) {
+    return kry_split(nsl) ? std::max(1, nsl) : row_blocks(1, nsl);
 }
 
 // lanes per field of the node-block SpMV: the node-graph degree (incl. the node itself)
@@ -566,8 +575,8 @@ void Engine::Impl::load_views(Req* r) {
         k.x_zero = 0;
         k.nodes = N;
         k.nf = dim + 1;
-        k.nblk = row_blocks(n, P.ell_nsl);
-        k.A = node_mat<double>(P, dim, w.vals);
+        k.nblk = kry_blocks(P.ell_nsl);
+        k.split = kry_split(P.ell_nsl);
         k.binv = w.binv;
         k.b = w.b;
         k.x = w.x;
@@ -581,19 +590,18 @@ void Engine::Impl::load_views(Req* r) {
         k.ph = v + 6 * n;
         k.sh = v + 7 * n;
         k.partials = c->partials.as<double>();
-        k.counters = c->counters.as<unsigned>();
         k.sc = &ds->k[0];
         k.E = ell_mat<double>(P, dim, w.vals_ell);
         k.amg = c->amg.levels > 1 ? 1 : 0;
         if (k.amg) {
-            if (amg_fp32(c))
+            if (amg_fp32(c)) {
                 load_amg<float>(c, slot, k, h_amg32, d_amg32, node_mat<float>(P, dim, w.vals32), w.binv32);
-            else {
+                k.mg_w0f = reinterpret_cast<float*>(w.amg_w0);
+            } else {
                 load_amg<double>(c, slot, k, h_amg64, d_amg64, node_mat<double>(P, dim, w.vals), w.binv);
-                // K_p / K_s write the level-0 pre-smoothing (the FP64 V-cycle launches none)
                 k.mg_w0 = reinterpret_cast<double*>(w.amg_w0);
-                k.mg_om = std::min(amg_omega, c->amg_omega_cap);
             }
+            k.mg_om = std::min(amg_omega, c->amg_omega_cap);
         }
 
         KrylovView<float>& f = h_k32[slot];
@@ -606,8 +614,8 @@ void Engine::Impl::load_views(Req* r) {
             f.x_zero = 1;
             f.nodes = N;
             f.nf = dim + 1;
-            f.nblk = row_blocks(n, P.ell_nsl);
-            f.A = node_mat<float>(P, dim, w.vals32);
+            f.nblk = kry_blocks(P.ell_nsl);
+            f.split = kry_split(P.ell_nsl);
             f.E = ell_mat<float>(P, dim, w.vals32_ell);  // the inner solve's SpMVs run over the FP32 ELL copy
             f.binv = w.binv32;
             f.b = u;
@@ -621,7 +629,6 @@ void Engine::Impl::load_views(Req* r) {
             f.ph = u + 8 * n;
             f.sh = u + 9 * n;
             f.partials = c->partials.as<double>();
-            f.counters = c->counters.as<unsigned>();
             f.sc = &ds->k[1];
             rv.n = (int)n;
             rv.A = node_mat<double>(P, dim, w.vals);
@@ -1055,10 +1062,13 @@ void Engine::tick(std::vector<Req*>& done) {
         }
         if (op & OP_IRU) append_rows(tab[T_IRU], sl, c->n, c->pat.ell_nsl);
         if (op & OP_IRR) append_rows(tab[T_IRR + li], sl, c->n, c->pat.ell_nsl);
-        if (op & OP_K64_RUN) append_rows(tab[T_K64 + li], sl, c->n, c->pat.ell_nsl);
-        if (op & OP_K32_RUN) append_rows(tab[T_K32 + li], sl, c->n, c->pat.ell_nsl);
-        if (op & OP_K64_INIT) tab[T_F64 + li].push_back(BlockTask{sl, 0, 1, 0});
-        if (op & OP_K32_INIT) tab[T_F32 + li].push_back(BlockTask{sl, 0, 1, 0});
+        const int nk = kry_blocks(c->pat.ell_nsl);
+        if (op & OP_K64_RUN)
+            for (int b = 0; b < nk; ++b) tab[T_K64].push_back(BlockTask{sl, b, nk, 0});
+        if (op & OP_K32_RUN)
+            for (int b = 0; b < nk; ++b) tab[T_K32].push_back(BlockTask{sl, b, nk, 0});
+        if (op & OP_K64_INIT) tab[T_F64].push_back(BlockTask{sl, 0, 1, 0});
+        if (op & OP_K32_INIT) tab[T_F32].push_back(BlockTask{sl, 0, 1, 0});
         const AmgHierarchy& H = c->amg;
         if (pspg_like(c) && H.levels > 1) {
             const int base = sl * kAmgMaxLevels;  // AmgView index of (slot, level 0)
@@ -1165,14 +1175,8 @@ void Engine::tick(std::vector<Req*>& done) {
         if (NT(T_IRR + li)) launch_ir_residual(kLanes[li], vref, T(T_IRR + li), NT(T_IRR + li), s);
     const KrylovView<double>* vk64 = I.d_k64.as<KrylovView<double>>();
     const KrylovView<float>* vk32 = I.d_k32.as<KrylovView<float>>();
-    for (int li = 0; li < 3; ++li) {
-        if (NT(T_F64 + li))
-            launch_kry_init<double>(kLanes[li], vk64, T(T_K64 + li), NT(T_K64 + li), T(T_F64 + li), NT(T_F64 + li),
-                                    I.par ^ 1, s);
-        if (NT(T_F32 + li))
-            launch_kry_init<float>(kLanes[li], vk32, T(T_K32 + li), NT(T_K32 + li), T(T_F32 + li), NT(T_F32 + li),
-                                   I.par ^ 1, s);
-    }
+    if (NT(T_F64)) launch_kry_init<double>(vk64, T(T_K64), NT(T_K64), T(T_F64), NT(T_F64), I.par ^ 1, s);
+    if (NT(T_F32)) launch_kry_init<float>(vk32, T(T_K32), NT(T_K32), T(T_F32), NT(T_F32), I.par ^ 1, s);
     // live SpMV timing: one request iterating alone
     int prof_w = -1, prof_before = 0;
     if (I.prof && nrun == 1) {
@@ -1192,8 +1196,7 @@ void Engine::tick(std::vector<Req*>& done) {
             if (!NT(TA + A_VN + l)) break;
             const int tr = TA + (l == 0 ? A_VN : A_VS) + l;
             // the pre-smoothing of levels >= 1 is part of the restriction from the finer level,
-            // that of level 0 in FP64 hierarchies part of K_p / K_s (KrylovView::mg_w0)
-            if (l == 0 && TA != T_AMG) launch_amg_pre(v, T(TA + A_VN + l), NT(TA + A_VN + l), which, s);
+            // that of level 0 part of BiCGSTAB's U and S (KrylovView::mg_w0)
             launch_amg_res(v, T(tr), NT(tr), which, s);
             launch_amg_restrict(v, T(TA + A_VR + l), NT(TA + A_VR + l), s);
         }
@@ -1205,18 +1208,17 @@ void Engine::tick(std::vector<Req*>& done) {
         vcycle_type(vamg64, T_AMG, which);
         vcycle_type(vamg32, T_AMG + A_N, which);
     };
+    const bool multigrid = NT(T_AMG + A_VC) + NT(T_AMG + A_N + A_VC) > 0;
     auto run_chunk = [&]() {
         for (int it = 0; it < chunk; ++it) {
             const int p = (I.par + it) & 1;
-            for (int phase = 0; phase < 5; ++phase) {
-                for (int li = 0; li < 3; ++li) {
-                    if (NT(T_K64 + li))
-                        launch_kry_phase<double>(phase, kLanes[li], vk64, T(T_K64 + li), NT(T_K64 + li), p, s,
-                                                 (phase == 1 && prof_w == 0) ? I.pev + 2 * it : nullptr);
-                    if (NT(T_K32 + li))
-                        launch_kry_phase<float>(phase, kLanes[li], vk32, T(T_K32 + li), NT(T_K32 + li), p, s,
-                                                (phase == 1 && prof_w == 1) ? I.pev + 2 * it : nullptr);
-                }
+            for (int phase = 0; phase < 4; ++phase) {
+                if (NT(T_K64) && (phase != 2 || multigrid))  // S belongs to the multigrid cases
+                    launch_kry_phase<double>(phase, vk64, T(T_K64), NT(T_K64), p, s,
+                                             (phase == 1 && prof_w == 0) ? I.pev + 2 * it : nullptr);
+                if (NT(T_K32) && phase != 2)
+                    launch_kry_phase<float>(phase, vk32, T(T_K32), NT(T_K32), p, s,
+                                            (phase == 1 && prof_w == 1) ? I.pev + 2 * it : nullptr);
                 if (phase == 0) vcycle(0);
                 if (phase == 2) vcycle(1);
             }

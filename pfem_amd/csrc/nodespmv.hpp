@@ -26,8 +26,9 @@ namespace pfem {
 constexpr int kMaxNf = 4;
 
 // y[s] = (A x) of row (i, s), s < nf; valid in every lane of the group.  The values may
-// be stored in a narrower type VT than the vectors (FP32 values, FP64 vectors and sums).
-template <int L, typename VT, typename T>
+// be stored in a narrower type VT than the vectors (FP32 values, FP64 vectors and sums).  x is
+// field-blocked (entry j + t N), or node-blocked (entry j nf + t) with NODE.
+template <int L, bool NODE = false, typename VT, typename T>
 __device__ __forceinline__ void node_spmv(const NodeMat<VT>& M, const T* __restrict__ x, long long i, int lane,
                                           T (&y)[kMaxNf]) {
     const int4 inf = M.info[i];
@@ -54,7 +55,7 @@ __device__ __forceinline__ void node_spmv(const NodeMat<VT>& M, const T* __restr
         const long long j = M.nbr_idx[nb + k];
         T xv[kMaxNf];
 #pragma unroll
-        for (int t = 0; t < kMaxNf; ++t) xv[t] = (t < nf) ? x[j + t * Nx] : T(0);
+        for (int t = 0; t < kMaxNf; ++t) xv[t] = (t < nf) ? x[NODE ? j * nf + t : j + t * Nx] : T(0);
 #pragma unroll
         for (int s = 0; s < kMaxNf; ++s) {
             T acc = y[s];
@@ -66,7 +67,7 @@ __device__ __forceinline__ void node_spmv(const NodeMat<VT>& M, const T* __restr
     if (lane == 0) {
 #pragma unroll
         for (int s = 0; s < kMaxNf; ++s)
-            if (s < nf && !full[s]) y[s] = (T)M.vals[rs[s]] * x[i + s * N];
+            if (s < nf && !full[s]) y[s] = (T)M.vals[rs[s]] * x[NODE ? i * nf + s : i + s * N];
     }
 #pragma unroll
     for (int s = 0; s < kMaxNf; ++s)

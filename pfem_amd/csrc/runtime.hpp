@@ -200,6 +200,10 @@ int64_t now_ns();
 // workgroups per case of the row launches (Krylov, residual, refinement); nsl = the
 // case's ELL slices (0: none)
 int row_blocks(long long n, int nsl = 0);
+// whether the wavefronts of a workgroup share each ELL slice in a case's BiCGSTAB launches, and
+// the workgroups of those launches
+bool kry_split(int nsl);
+int kry_blocks(int nsl);
 int pick_lanes(double avg_deg);
 
 }  // namespace pfem

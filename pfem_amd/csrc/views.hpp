@@ -120,8 +120,11 @@ using EllMat = EllMatT<double>;
 // the current slot and only reads the previous one or fields written by earlier kernels,
 // so no workgroup ever reads a value another workgroup of the same launch is writing.
 struct KSlot {
-    double rho, alpha, omega, pad;
+    double rho, alpha, omega;
+    int state, pad;  // K_*: what the iteration's first kernel found
 };
+// Slot states: an iteration follows; the slot of a (re)start; converged on ||s||; breakdown.
+enum : int { K_RUN = 0, K_FRESH = 1, K_CONV = 2, K_BREAK = 3 };
 struct KScal {
     KSlot slot[2];
     double rr;    // last ||r||^2
@@ -137,36 +140,38 @@ struct KScal {
     int pad;
 };
 
-// Slots of the per-workgroup partial sums (kPartStride doubles per workgroup).
-enum : int { P_RHR = 0, P_RR = 1, P_RV = 2, P_SS = 3, P_TS = 4, P_TT = 5, P_BB = 6, kPartStride = 8 };
+// The per-workgroup partial sums: kPartStride arrays of kMaxCaseBlocks doubles per case.
+enum : int { P_RR = 0, P_RV = 1, P_SS = 2, P_TS = 3, P_TT = 4, P_RHT = 5, P_RHS = 6, P_RHR = 2, P_BB = 3, kPartStride = 8 };
 
 // BiCGSTAB workspace of one case; T is the inner arithmetic type (double or float).
-// Rows are n = nf * nodes (field-blocked); workgroups are assigned XCD-local node ranges.
+// x and b are field-blocked (entry f N + i) as the assembly and the Picard loop hold them, the
+// solver's own vectors node-blocked (entry i nf + f): a product gathers a neighbour's fields from
+// one cache line.  Workgroups are assigned XCD-local node ranges.
 template <typename T>
 struct KrylovView {
     int n, x_zero;
     int nodes, nf;
     int nblk;       // workgroups of this case in the Krylov launches (partials producers)
-    int amg;        // 1: ph and sh come from the multigrid V-cycle (K_p / K_s leave them)
-    NodeMat<T> A;
-    EllMatT<T> E;   // the ELL copy of A in type T used by K_v / K_t (vals null: node-block A)
+    int amg;        // 1: ph and sh come from the multigrid V-cycle
+    int split, pad_split;  // 1: the wavefronts of a workgroup share each slice of the products
+    EllMatT<T> E;   // the system's values in type T
     Gp<const T> binv;  // [nf*nf][nodes] inverse of each node's diagonal (nf x nf) block, SoA
     Gp<const T> b;
     Gp<T> x;
     Gp<T> r;
     Gp<T> rh;
-    Gp<T> p;
+    Gp<T> p;   // multigrid: p; block Jacobi: rhat = B^-1 r
     Gp<T> v;
-    Gp<T> s;
+    Gp<T> s;   // multigrid: s; block Jacobi: vhat = B^-1 v
     Gp<T> t;
     Gp<T> ph;
-    Gp<T> sh;
-    Gp<double> partials;    // [kMaxCaseBlocks * kPartStride]
-    Gp<unsigned> counters;  // [8]
+    Gp<T> sh;  // multigrid only
+    Gp<double> partials;    // [kPartStride][kMaxCaseBlocks]
     Gp<KScal> sc;
-    // FP64 multigrid: K_p / K_s also write the V-cycle's level-0 pre-smoothing w = om B^-1 p
-    // (or s) from the vector they hold (null: the V-cycle's own pre-smoothing launch does it)
+    // multigrid: U and S also write the V-cycle's level-0 pre-smoothing w = om B^-1 p (or s) from
+    // the vector they hold, in the hierarchy's type
     Gp<double> mg_w0;
+    Gp<float> mg_w0f;
     double mg_om;
 };
 
@@ -231,7 +236,7 @@ struct AmgView {
     Gp<const int> self_rank;
     Gp<T> vals_out;
     Gp<T> binv_out;
-    Gp<double> dense;  // coarsest: [nc * nc] inverse, row major over unknowns I + s N (FP64 in
+    Gp<double> dense;  // coarsest: [nc * nc] inverse, row major over unknowns I nf + s (FP64 in
                     // either type: the coarse operators are the worst conditioned)
 };
 
