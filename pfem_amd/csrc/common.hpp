@@ -175,7 +175,8 @@ __device__ __forceinline__ void gj_invert4(double (&m)[4][8]) {
 
 // Smallest positive value over the workgroup folded into *addr (the bits of a positive
 // double, compared as integers): one atomic per workgroup, since every atomic on one address
-// is serialised (one per wavefront cost ~10 ns each, 0.3 ms over 2M nodes).
+// is serialised (~10 ns each: 0.3 ms over 2M nodes with one per wavefront), and none where the
+// minimum already stands below (it only falls, so an old value read here costs one atomic more).
 __device__ __forceinline__ void block_min_to(unsigned long long* addr, double v) {
     __shared__ double red[kWaves];
     v = wave_min(v);
@@ -185,7 +186,8 @@ __device__ __forceinline__ void block_min_to(unsigned long long* addr, double v)
         double m = red[0];
 #pragma unroll
         for (int w = 1; w < kWaves; ++w) m = fmin(m, red[w]);
-        atomicMin(addr, (unsigned long long)__double_as_longlong(m));
+        const unsigned long long b = (unsigned long long)__double_as_longlong(m);
+        if (b < __hip_atomic_load(addr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(addr, b);
     }
 }
 

@@ -658,6 +658,7 @@ void Engine::Impl::load_views(Req* r) {
             V.elem_ptr = c->pat.elem_ptr.as<int>();
             V.elem_list = c->pat.elem_list.as<uint32_t>();
             V.ntiles = c->pat.ntiles;
+            V.lanes = c->pat.tile_lanes;
             V.tile_own = c->pat.tile_own.as<int>();
             V.tile_nodes = c->pat.tile_nodes.as<int>();
             V.visit = c->pat.visit.as<uint32_t>();

@@ -40,8 +40,8 @@ struct Pattern {
     // elem_ptr[i] .. elem_ptr[i+1] hold e << 2 | a with conn[e][a] = i, sorted by element
     DevBuf elem_ptr;   // int  [N + 1]
     DevBuf elem_list;  // u32  [E * ne]
-    // tiles of the weakly compressible passes (kWcTile nodes each; views.hpp)
-    int ntiles = 0, tile_max = 0;  // tiles, most nodes staged by one
+    // tiles of the weakly compressible passes (kBlock / tile_lanes nodes each; views.hpp)
+    int ntiles = 0, tile_max = 0, tile_lanes = 0;  // tiles, most nodes staged by one, lanes per node
     DevBuf tile_own;   // int  [ntiles] slot of the tile's first node
     DevBuf tile_nodes; // int  [ntiles][kWcTileCap] staged nodes, ascending, then -1
     DevBuf visit;      // u32  [E * ne] slots of the other nodes of each incidence entry (10 bits

@@ -262,6 +262,7 @@ struct RefineView {
 // through memory (kWcFar), visit words past theirs are read from memory.
 constexpr int kWcTile[2] = {128, 64};
 constexpr int kWcTileLanes[2] = {2, 4};
+constexpr int kWcSmallLanes[2] = {2, 16};  // of small cases (build_mesh_basic): kBlock / lanes nodes per tile
 constexpr int kWcTileCap = 752;
 constexpr int kWcVisits[2] = {1024, 1792};
 constexpr uint32_t kWcFar = 0xffffffffu;
@@ -281,7 +282,7 @@ struct WcView {
     Gp<const uint8_t> flags;     // [N] with NODE_FREE derived
     Gp<const int> elem_ptr;        // [N+1] node-element incidence (Pattern::elem_ptr / elem_list)
     Gp<const uint32_t> elem_list;
-    int ntiles, pad_tiles;
+    int ntiles, lanes;
     Gp<const int> tile_own;      // [ntiles] LDS slot of the tile's first node
     Gp<const int> tile_nodes;    // [ntiles][kWcTileCap] staged nodes, ascending, then -1
     Gp<const uint32_t> visit;    // per incidence entry: LDS slots of the other nodes, 10 bits each, or kWcFar

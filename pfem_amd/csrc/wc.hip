@@ -8,9 +8,9 @@
 // finish their nodes).  There are no atomics on sums: device-scope FP64 atomics on gfx950 ran
 // at ~36 G/s; every sum is gathered per node in a fixed order.
 //
-// Tile passes.  A workgroup owns kWcTile consecutive nodes.  The nodes of all their elements
-// (the tile's nodes and a halo, listed once per mesh) are staged in LDS, and kWcTileLanes
-// lanes per node walk the node's incident elements, finding each element's other nodes through
+// Tile passes.  A workgroup owns kWcTile consecutive nodes (small 3D cases: 16).  The nodes of
+// all their elements (the tile's nodes and a halo, listed once per mesh) are staged in LDS, and
+// kWcTileLanes (16) lanes per node walk the node's incident elements, finding each element's other nodes through
 // one 32-bit word of LDS slots (WcView::visit).  Reading the nodes from memory at every visit
 // (d x 64 bytes, 24 visits per node in 3D) was bound by the rate at which the L1 looks up
 // scattered cache lines: the 3D momentum gather took the same time per visit on a mesh that
@@ -18,7 +18,7 @@
 // ~7 node states per node instead of 72, mostly in runs.  On the 2.06M-node 3D tank (12M tets,
 // FP32 state) the six kernels of the record gathers (half 82, continuity element pass 280 and
 // gather 255, node pass 56, momentum gather 767, node pass 78 us) became half 34, continuity 379
-// and momentum 369 us; 100k nodes in FP64: 88 -> 62 us.  What bounds the tile passes now is FP64
+// and momentum 369 us; 100k nodes in FP64: 88 -> 60 us.  What bounds the tile passes now is FP64
 // issue (a visit is ~165 vector instructions in 3D, 200 us of the 369 at the full rate) and,
 // behind it, the latency of staging with four workgroups per CU.
 //
@@ -172,8 +172,9 @@ struct TileLds {
     }
     // Every thread takes all its list entries, then all their states, so that staging costs a few
     // memory latencies in all and not a few per record.
+    template <int T>
     __device__ __forceinline__ void stage(const WcView<S>& V, const S* __restrict__ pin, int tile) {
-        constexpr int T = kWcTile[D - 2], kVis = kWcVisits[D - 2];
+        constexpr int kVis = kWcVisits[D - 2];
         constexpr int R = (kWcTileCap + kBlock - 1) / kBlock, RV = kVis / kBlock;
         static_assert(kVis % kBlock == 0, "whole rounds of visit words");
         const int* __restrict__ list = V.tile_nodes + (long long)tile * kWcTileCap;
@@ -203,6 +204,7 @@ struct TileLds {
         uint32_t w[RV];
 #pragma unroll
         for (int r = 0; r < RV; ++r) {
+            if (r * kBlock >= q1 - q0) continue;  // (uniform)
             const int q = q0 + (int)threadIdx.x + r * kBlock;
             w[r] = V.visit[max(min(q, q1 - 1), 0)];  // past the tile: unused
         }
@@ -219,7 +221,10 @@ struct TileLds {
             if (MOM) u[k * kU + D + 1] = rs[r];
         }
 #pragma unroll
-        for (int r = 0; r < RV; ++r) words[(int)threadIdx.x + r * kBlock] = w[r];
+        for (int r = 0; r < RV; ++r) {
+            if (r * kBlock >= q1 - q0) continue;
+            words[(int)threadIdx.x + r * kBlock] = w[r];
+        }
     }
     __device__ __forceinline__ void get(int k, double (&xa)[D], double (&va)[D], double& pa, double& ra) const {
 #pragma unroll
@@ -287,16 +292,10 @@ __device__ __forceinline__ void visit_elem(const WcView<S>& V, const TileLds<D, 
 // Continuity (m_buildSystemdpdt, ContEquation.inl:353-413, 139-147, 319-350): lumped mass
 // lump2(M(1)), rhs F0 = -dt D(K0 + K0' N.P) V + M(1) P (Meduri) or lump2(M(1)) P and the
 // smallest he of each node, then p = M^-1 F0 (free nodes: 0) and rho from the Tait-Murnaghan law.
-template <int D, typename S>
-__global__ __launch_bounds__(kBlock, 4) void k_wc_cont(const WcView<S>* __restrict__ views,
-                                                    const BlockTask* __restrict__ tasks, int cap) {
-    constexpr int L = kWcTileLanes[D - 2], T = kWcTile[D - 2];
-    static_assert(L * T == kBlock, "a lane group per tile node");
-    extern __shared__ double lds[];
-    __shared__ double red[2][T];
-    const BlockTask task = tasks[blockIdx.x];
-    if (task.case_id < 0) return;
-    const WcView<S>& V = views[task.case_id];
+template <int D, typename S, int L>
+__device__ __forceinline__ void wc_cont_tiles(const WcView<S>& V, const BlockTask& task, int cap, double* lds,
+                                              double (&red)[2][kWcTile[D - 2]]) {
+    constexpr int T = kBlock / L;  // a lane group per tile node
     const int N = V.N;
     const double dt = V.dt;
     const int lane = threadIdx.x % L, r = threadIdx.x / L;
@@ -310,7 +309,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_wc_cont(const WcView<S>* __restri
         const uint8_t fl = fin ? V.flags[j] : (uint8_t)0;
         const int i = tile * T + r;
         const int qb = i < N ? V.elem_ptr[i] : 0, qe = i < N ? V.elem_ptr[i + 1] : 0;
-        TL.stage(V, V.p_old, tile);
+        TL.template stage<T>(V, V.p_old, tile);
         __syncthreads();
         double ml = 0.0, fc = 0.0, hmin = 1.7976931348623157e308;
         if (i < N) {
@@ -352,6 +351,19 @@ __global__ __launch_bounds__(kBlock, 4) void k_wc_cont(const WcView<S>* __restri
     }
 }
 
+template <int D, typename S>
+__global__ __launch_bounds__(kBlock, 4) void k_wc_cont(const WcView<S>* __restrict__ views,
+                                                    const BlockTask* __restrict__ tasks, int cap) {
+    extern __shared__ double lds[];
+    __shared__ double red[2][kWcTile[D - 2]];
+    const BlockTask task = tasks[blockIdx.x];
+    if (task.case_id < 0) return;
+    const WcView<S>& V = views[task.case_id];
+    if (kWcSmallLanes[D - 2] == kWcTileLanes[D - 2] || V.lanes == kWcTileLanes[D - 2])
+        wc_cont_tiles<D, S, kWcTileLanes[D - 2]>(V, task, cap, lds, red);
+    else wc_cont_tiles<D, S, kWcSmallLanes[D - 2]>(V, task, cap, lds, red);
+}
+
 // The end of a step at node i: a = M^-1 F with the BC of MomEquation.inl:341-373,
 // v = v1/2 + dt/2 a (:216-222), and the node's share of the next step's CFL time step from the
 // final v, p, rho and its smallest incident he (free nodes belong to no element: no share).
@@ -383,15 +395,10 @@ __device__ __forceinline__ double wc_finish(const WcView<S>& V, int i, uint8_t f
 // with w_a = v_a - v_i, c_a and C of Frame, grad v = sum_a w_a c_a^T / dj and grad N_i = -C / dj:
 //   (K V)_i = -mu refSize / dj [ sum_a (w_a (c_a.C) + c_a (w_a.C)) - 2/3 (sum_a w_a.c_a) C ].
 // Cases with surface-tension facets leave the sums for k_wc_mom_node, which adds the facet terms.
-template <int D, typename S>
-__global__ __launch_bounds__(kBlock, 4) void k_wc_mom(const WcView<S>* __restrict__ views,
-                                                   const BlockTask* __restrict__ tasks, int cap) {
-    constexpr int L = kWcTileLanes[D - 2], T = kWcTile[D - 2];
-    extern __shared__ double lds[];
-    __shared__ double red[D + 1][T];
-    const BlockTask task = tasks[blockIdx.x];
-    if (task.case_id < 0) return;
-    const WcView<S>& V = views[task.case_id];
+template <int D, typename S, int L>
+__device__ __forceinline__ void wc_mom_tiles(const WcView<S>& V, const BlockTask& task, int cap, double* lds,
+                                              double (&red)[D + 1][kWcTile[D - 2]]) {
+    constexpr int T = kBlock / L;  // a lane group per tile node
     const int N = V.N;
     const double c2 = 1.0 / (double)((D + 1) * (D + 2));
     const double muf = V.mu * (D + 1);  // in units of refSize / (d + 1)
@@ -408,7 +415,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_wc_mom(const WcView<S>* __restric
         const double hmin = fin ? V.hmin[j] : 0.0;
         const int i = tile * T + r;
         const int qb = i < N ? V.elem_ptr[i] : 0, qe = i < N ? V.elem_ptr[i + 1] : 0;
-        TL.stage(V, V.p, tile);
+        TL.template stage<T>(V, V.p, tile);
         __syncthreads();
         if (i < N) {
             double x0[D], v0[D], p0, r0, mm = 0.0, fm[D];
@@ -467,6 +474,19 @@ __global__ __launch_bounds__(kBlock, 4) void k_wc_mom(const WcView<S>* __restric
         __syncthreads();
     }
     if (V.fst.F == 0) block_min_to(V.dt2, best);
+}
+
+template <int D, typename S>
+__global__ __launch_bounds__(kBlock, 4) void k_wc_mom(const WcView<S>* __restrict__ views,
+                                                    const BlockTask* __restrict__ tasks, int cap) {
+    extern __shared__ double lds[];
+    __shared__ double red[D + 1][kWcTile[D - 2]];
+    const BlockTask task = tasks[blockIdx.x];
+    if (task.case_id < 0) return;
+    const WcView<S>& V = views[task.case_id];
+    if (kWcSmallLanes[D - 2] == kWcTileLanes[D - 2] || V.lanes == kWcTileLanes[D - 2])
+        wc_mom_tiles<D, S, kWcTileLanes[D - 2]>(V, task, cap, lds, red);
+    else wc_mom_tiles<D, S, kWcSmallLanes[D - 2]>(V, task, cap, lds, red);
 }
 
 // The end of the step for cases with surface-tension facets: the force with the FST entries of

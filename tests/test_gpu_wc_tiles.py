@@ -1,7 +1,8 @@
 """The tile passes of the weakly compressible step against the oracle where their tiles are at
 their limits: node counts around whole tiles, nodes numbered at random (a tile then refers to
 more nodes than it stages, so elements are visited through memory), a node with more elements
-than a tile's staged visit words, and nodes in no element.
+than a tile's staged visit words, nodes in no element, and 3D cases on both sides of the size
+(16,384 nodes) up to which tiles are small.
 
 Tolerance: the FP64 step differs from the oracle by the rounding of its sums and of a handful of
 products per element, a few hundred ulp (1e-13) of the largest term; the pressure terms that
@@ -50,6 +51,7 @@ CASES = {
     "2d_random_order": lambda: renumber(mg.tank_nodes(2, 3000), 1), "2d_fan_1200": lambda: fan(1200),
     "3d_small": lambda: mg.tank_3d(h=0.5, size=(1.0, 1.0, 1.0), fill=1.0),
     "3d_random_order": lambda: renumber(mg.tank_nodes(3, 4000), 2),
+    "3d_large_tiles_random_order": lambda: renumber(mg.tank_nodes(3, 20000), 2),
 }
 
 
