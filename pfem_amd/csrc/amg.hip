@@ -8,13 +8,18 @@
 //   w = omega B^-1 r                      (block-Jacobi pre-smoothing: at level 0 done by the
 //                                          BiCGSTAB kernel that forms r_0, on coarser levels by
 //                                          the restriction above)
-//   t = r - A w                           (k_amg_res)
-//   r_{l+1} = P^T t                       (k_amg_restrict, gather over aggregate members)
-//   z_{l+1} = V-cycle(l+1)  /  A_c^-1 r_c (k_amg_coarsest, dense inverse on the coarsest)
+//   t = r - A w                           (k_amg_res; levels >= 1: k_amg_rr)
+//   r_{l+1} = P^T t                       (k_amg_restrict, gather over aggregate members; k_amg_rr)
+//   z_{l+1} = V-cycle(l+1)  /  A_c^-1 r_c (k_amg_tail, dense inverse on the coarsest)
 //   w' = w + alpha P z_{l+1}              (alpha > 1 over-corrects the piecewise-constant
 //                                          interpolation)
 //   z = w' + omega B^-1 (r - A w')        (k_amg_post, post-smoothing; r - A w' is formed
 //       = w' + omega B^-1 (t - alpha (A P) z_{l+1})   from t with the set-up product A P)
+// Every vector of the cycle is node-blocked (entry i nf + s), as BiCGSTAB's are.
+// What bounds it: on level 0 the matrix's bytes (large cases), elsewhere a chain of dependent loads
+// of 4-6 us per launch.  With a launch of its own for every residual, restriction and solve a
+// V-cycle took 13 launches and 48 us on 20k nodes in 2D (five levels), now 8 and 37 us; on 263k nodes
+// in 3D 141 -> 131 us.
 // Every reduction is a fixed-order gather, so a case's V-cycle does not depend on the batch.
 #include <type_traits>
 
@@ -35,12 +40,7 @@ __device__ __forceinline__ long long row_start_of(const int4& inf, int s, int D,
     return (s < D) ? (long long)s * mom_nnz + inf.x : (long long)D * mom_nnz + inf.y;
 }
 
-// Entry q of the level's input (level 0: the FP64 Krylov vector p or s); every vector of the
-// V-cycle is node-blocked (entry i nf + s), as BiCGSTAB's are.
-template <typename T>
-__device__ __forceinline__ T in_at(const AmgView<T>& V, int which, long long q) {
-    return V.level == 0 ? (T)V.r0[which][q] : V.r[q];
-}
+constexpr int kTailBlock = 1024;
 
 }  // namespace
 
@@ -300,67 +300,102 @@ __global__ __launch_bounds__(kBlock) void k_amg_dense(const AmgView<T>* __restri
 
 // ---- V-cycle -----------------------------------------------------------------------------
 
-template <typename T, int L>
-__device__ __forceinline__ void res_body(const AmgView<T>& V, const BlockTask& task, int which) {
-    constexpr int NPB = kBlock / L;
-    const int lane = threadIdx.x % L;
-    const int N = V.A.N;
-    for (long long i = (long long)task.block * NPB + threadIdx.x / L; i < N; i += (long long)task.nblocks * NPB) {
-        T y[kMaxNf];
-        node_spmv<L, true>(V.A, (const T*)V.w, i, lane, y);
-        if (lane < V.A.nf) {
-            const long long q = i * V.A.nf + lane;
-            V.t[q] = in_at(V, which, q) - pick(y, lane);
-        }
-    }
+// Level 0, over the system's ELL copy; an FP64 hierarchy reads the FP32 copy of the values when
+// the view has one (E0f).
+template <int NF, int MODE, typename T>
+__device__ __forceinline__ void res_rows(const AmgView<T>& V, const BlockTask& task, int which) {
+    auto xat = [&](long long j, T (&xv)[NF]) { at_node<NF>((const T*)V.w, j, xv); };
+    auto prod = [&](long long c, int k0, int step, T (&acc)[NF]) {
+        if (V.E0f.vals) slice_part<NF, (MODE & ELL_STREAM) != 0>(V.E0f, c, k0, step, xat, acc);
+        else slice_part<NF, (MODE & ELL_STREAM) != 0>(V.E0, c, k0, step, xat, acc);
+    };
+    auto pre = [&](long long i, int f) { return (T)V.r0[which][i * NF + f]; };
+    auto fin = [&](long long i, int f, const T (&y)[NF], T r, int h) {
+        if (!h) V.t[i * NF + f] = r - at_field(y, f);
+    };
+    slice_products<NF, MODE, T>(task, V.E0.nsl, V.E0.N, prod, pre, fin);
 }
 
-// Level 0 with the system's ELL copy: one lane per node, whole 64-node slices per
-// wavefront (a workgroup's waves stride over the case's slices); an FP64 hierarchy reads
-// the FP32 copy of the values when the view has one (E0f).
-template <int NF, typename T>
-__device__ __forceinline__ void res_ell(const AmgView<T>& V, const BlockTask& task, int which) {
-    const EllMatT<T>& E = V.E0;
-    const int lane = threadIdx.x & (kEllSlice - 1);
-    const long long N = E.N;
-    for (long long c = (long long)task.block * kWaves + (threadIdx.x >> 6); c < E.nsl;
-         c += (long long)task.nblocks * kWaves) {
-        T y[NF];
-        auto xat = [&](long long j, T (&xv)[NF]) { at_node<NF>((const T*)V.w, j, xv); };
-        if (V.E0f.vals) slice_part<NF>(V.E0f, c, 0, 1, xat, y);
-        else slice_part<NF>(E, c, 0, 1, xat, y);
-        const long long i = c * kEllSlice + lane;
-        if (i < N) {
-#pragma unroll
-            for (int s = 0; s < NF; ++s) {
-                const long long q = i * NF + s;
-                V.t[q] = (T)V.r0[which][q] - y[s];
-            }
-        }
-    }
-}
-
-template <typename T>
+template <typename T, bool STREAM>
 __global__ __launch_bounds__(kBlock) void k_amg_res(const AmgView<T>* __restrict__ views,
                                                     const BlockTask* __restrict__ tasks, int which) {
     const BlockTask task = tasks[blockIdx.x];
     if (task.case_id < 0) return;
     const AmgView<T>& V = views[task.case_id];
     if (*V.done_flag) return;
-    if (V.level == 0 && V.E0.vals) {
-        if (V.A.nf == 4) res_ell<4>(V, task, which);
-        else res_ell<3>(V, task, which);
-        return;
-    }
-    if (V.lanes == 4) res_body<T, 4>(V, task, which);
-    else if (V.lanes == 8) res_body<T, 8>(V, task, which);
-    else res_body<T, 16>(V, task, which);
+    PFEM_NF_MODE(res_rows, STREAM, V.A.nf, V.split, V, task, which);
 }
 
-// r_{l+1}(I, s) = sum over the members i of aggregate I of t(i, s) (level 0: full rows only);
+// Residual and restriction of a level l >= 1 in one pass, a workgroup per aggregate: its lane
+// groups take the aggregate's members (every node of a coarse level has an aggregate), form
+// t = r - A w there and sum it per group in member order, then over the groups.  When level l+1
+// is not the coarsest its pre-smoothing follows, as in k_amg_restrict.
+template <typename T, int L>
+__device__ __forceinline__ void rr_body(const AmgView<T>& V, const AmgView<T>& Vn, const BlockTask& task,
+                                        double (&red)[kWaves][kMaxNf]) {
+    const int lane = threadIdx.x % L, wl = threadIdx.x & 63, nf = V.A.nf, Nc = V.next_N;
+    const bool smooth = Vn.dense == nullptr;
+    for (int I = task.block; I < Nc; I += task.nblocks) {
+        double acc[kMaxNf] = {0.0, 0.0, 0.0, 0.0};
+        for (int m = V.agg_ptr[I] + (int)threadIdx.x / L; m < V.agg_ptr[I + 1]; m += kBlock / L) {
+            const long long i = V.agg_nodes[m];
+            T y[kMaxNf];
+            node_spmv<L, true>(V.A, (const T*)V.w, i, lane, y);
+#pragma unroll
+            for (int s = 0; s < kMaxNf; ++s)
+                if (s < nf) {
+                    y[s] = V.r[i * nf + s] - y[s];
+                    acc[s] += (double)y[s];
+                }
+            if (lane < nf) V.t[i * nf + lane] = pick(y, lane);
+        }
+#pragma unroll
+        for (int s = 0; s < kMaxNf; ++s) {
+#pragma unroll
+            for (int o = L; o < 64; o <<= 1) acc[s] += __shfl_xor(acc[s], o, 64);
+            if (wl == 0) red[threadIdx.x >> 6][s] = acc[s];
+        }
+        __syncthreads();
+        if ((int)threadIdx.x < nf) {
+            double sum[kMaxNf];
+#pragma unroll
+            for (int s = 0; s < kMaxNf; ++s) {
+                sum[s] = red[0][s];
+#pragma unroll
+                for (int w = 1; w < kWaves; ++w) sum[s] += red[w][s];
+            }
+            const int f = threadIdx.x;
+            V.next_r[(long long)I * nf + f] = (T)pick(sum, f);
+            if (smooth) {
+                T w = 0;
+#pragma unroll
+                for (int t = 0; t < kMaxNf; ++t)
+                    if (t < nf) w += Vn.binv[(long long)(f * nf + t) * Nc + I] * (T)sum[t];
+                Vn.w[(long long)I * nf + f] = (T)Vn.omega * w;
+            }
+        }
+        __syncthreads();
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_amg_rr(const AmgView<T>* __restrict__ views,
+                                                   const BlockTask* __restrict__ tasks) {
+    const BlockTask task = tasks[blockIdx.x];
+    if (task.case_id < 0) return;
+    const AmgView<T>& V = views[task.case_id];
+    if (*V.done_flag) return;
+    const AmgView<T>& Vn = views[task.case_id + 1];  // level l+1 (views of a case are consecutive)
+    __shared__ double red[kWaves][kMaxNf];
+    if (V.lanes == 4) rr_body<T, 4>(V, Vn, task, red);
+    else if (V.lanes == 8) rr_body<T, 8>(V, Vn, task, red);
+    else rr_body<T, 16>(V, Vn, task, red);
+}
+
+// Level 0: r_1(I, s) = sum over the members i of aggregate I of t(i, s) (full rows only);
 // kRestrictLanes lanes per aggregate share its members (aggregates hold 5-30 nodes).  When
-// level l+1 is not the coarsest, its pre-smoothing w_{l+1}(I) = omega B^-1(I) r_{l+1}(I) is
-// local to I and is applied here as well.
+// level 1 is not the coarsest, its pre-smoothing w_1(I) = omega B^-1(I) r_1(I) is local to I and
+// is applied here as well.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_amg_restrict(const AmgView<T>* __restrict__ views,
                                                          const BlockTask* __restrict__ tasks) {
@@ -399,67 +434,139 @@ __global__ __launch_bounds__(kBlock) void k_amg_restrict(const AmgView<T>* __res
     }
 }
 
-// z = A_c^-1 r on the coarsest level (one workgroup per case).
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_amg_coarsest(const AmgView<T>* __restrict__ views,
-                                                         const BlockTask* __restrict__ tasks) {
-    const BlockTask task = tasks[blockIdx.x];
-    if (task.case_id < 0) return;
-    const AmgView<T>& V = views[task.case_id];
-    if (*V.done_flag) return;
-    const int n = V.nc;
-    for (int row = threadIdx.x; row < n; row += kBlock) {
-        double acc = 0.0;
-        for (int j = 0; j < n; ++j) acc += V.dense[row * n + j] * (double)V.r[j];
-        V.z[row] = (T)acc;
+// The end of the V-cycle in one workgroup per case: on the coarsest level z = A_c^-1 r (8 lanes
+// per unknown), and with task.pad the level above it too (kAmgTailNodes), its residual and
+// restriction before and its post-smoothing after, with t, r_c and z_c in LDS.
+template <typename T, int L>
+__device__ __forceinline__ void tail_down(const AmgView<T>& V, T* __restrict__ tl, double* __restrict__ rc) {
+    const int lane = threadIdx.x % L, nf = V.A.nf;
+    for (int i = threadIdx.x / L; i < V.A.N; i += kTailBlock / L) {
+        T y[kMaxNf];
+        node_spmv<L, true>(V.A, (const T*)V.w, i, lane, y);
+        if (lane < nf) tl[i * nf + lane] = V.r[(long long)i * nf + lane] - pick(y, lane);
     }
+    __syncthreads();
+    for (int k = threadIdx.x; k < V.next_N * nf; k += kTailBlock) {
+        const int I = k / nf, f = k - I * nf;
+        double acc = 0.0;
+        for (int m = V.agg_ptr[I]; m < V.agg_ptr[I + 1]; ++m) acc += (double)tl[V.agg_nodes[m] * nf + f];
+        rc[k] = (double)(T)acc;
+    }
+    __syncthreads();
 }
 
-// z = w' + omega B^-1 (t - alpha (A P) z_{l+1}),  w' = w + alpha P z_{l+1} (level 0: full
-// rows only): one lane per node, whole 64-node slices per wavefront; A P in FP32 when the
-// view holds it so (APf).
-template <int NF, typename T>
-__device__ __forceinline__ void post_ell(const AmgView<T>& V, const BlockTask& task, int which) {
-    const int N = V.A.N, D = NF - 1;
+template <typename T, int L>
+__device__ __forceinline__ void tail_up(const AmgView<T>& V, const T* __restrict__ tl, const T* __restrict__ zc) {
+    const int lane = threadIdx.x % L, nf = V.A.nf, N = V.A.N;
     const T om = (T)V.omega, al = (T)V.alpha;
-    const int lane = threadIdx.x & (kEllSlice - 1);
-    for (long long c = (long long)task.block * kWaves + (threadIdx.x >> 6); c < V.AP.nsl;
-         c += (long long)task.nblocks * kWaves) {
-        T y[NF];
-        auto xat = [&](long long j, T (&xv)[NF]) { at_node<NF>(V.next_z.get(), j, xv); };
-        if (V.APf.vals) slice_part<NF>(V.APf, c, 0, 1, xat, y);
-        else slice_part<NF>(V.AP, c, 0, 1, xat, y);
-        const long long i = c * kEllSlice + lane;
-        if (i >= N) continue;
-        T d[NF];
+    for (int i = threadIdx.x / L; i < N; i += kTailBlock / L) {
+        const int c = i / kEllSlice, r = i % kEllSlice, b = V.AP.soff[c], W = V.AP.soff[c + 1] - b;
+        T y[kMaxNf] = {T(0), T(0), T(0), T(0)};
+        for (int k = lane; k < W; k += L) {
+            const int J = V.AP.idx[(long long)(b + k) * kEllSlice + r];
+            const T* __restrict__ a = V.AP.vals + (long long)(b + k) * nf * nf * kEllSlice + r;
 #pragma unroll
-        for (int t = 0; t < NF; ++t) d[t] = V.t[i * NF + t] - al * y[t];
-        const int I = V.fine_agg[i];
-        const uint8_t f = V.mask ? V.flags[i] : (uint8_t)0;
+            for (int s = 0; s < kMaxNf; ++s)
 #pragma unroll
-        for (int s = 0; s < NF; ++s) {
+                for (int t = 0; t < kMaxNf; ++t)
+                    if (s < nf && t < nf) y[s] += a[(long long)(s * nf + t) * kEllSlice] * zc[J * nf + t];
+        }
+        T d[kMaxNf];
+#pragma unroll
+        for (int s = 0; s < kMaxNf; ++s) d[s] = s < nf ? tl[i * nf + s] - al * group_sum<L>(y[s]) : T(0);
+        if (lane < nf) {
             T acc = 0;
 #pragma unroll
-            for (int t = 0; t < NF; ++t) acc += V.binv[(long long)(s * NF + t) * N + i] * d[t];
-            const long long q = i * NF + s;
-            T wq = V.w[q];
-            if (I >= 0 && (!V.mask || row_full_flags(f, s, D))) wq += al * V.next_z[(long long)I * NF + s];
-            const T out = wq + om * acc;
-            if (V.level == 0) V.out0[which][q] = (double)out;
-            else V.z[q] = out;
+            for (int t = 0; t < kMaxNf; ++t)
+                if (t < nf) acc += V.binv[(long long)(lane * nf + t) * N + i] * d[t];
+            const long long q = (long long)i * nf + lane;
+            V.z[q] = V.w[q] + al * zc[V.fine_agg[i] * nf + lane] + om * acc;
         }
     }
 }
 
 template <typename T>
+__global__ __launch_bounds__(kTailBlock) void k_amg_tail(const AmgView<T>* __restrict__ views,
+                                                         const BlockTask* __restrict__ tasks) {
+    __shared__ T tl[kAmgTailNodes * kMaxNf];
+    __shared__ double rc[kAmgMaxDense];
+    __shared__ T zc[kAmgMaxDense];
+    const BlockTask task = tasks[blockIdx.x];
+    if (task.case_id < 0) return;
+    const AmgView<T>& V = views[task.case_id];
+    if (*V.done_flag) return;
+    const int n = V.nc;
+    const AmgView<T>& Vf = views[task.case_id - task.pad];  // the level above
+    if (task.pad) {
+        if (Vf.lanes == 4) tail_down<T, 4>(Vf, tl, rc);
+        else if (Vf.lanes == 8) tail_down<T, 8>(Vf, tl, rc);
+        else tail_down<T, 16>(Vf, tl, rc);
+    } else {
+        for (int k = threadIdx.x; k < n; k += kTailBlock) rc[k] = (double)V.r[k];
+        __syncthreads();
+    }
+    const int lane = threadIdx.x % 8;
+    for (int row = threadIdx.x / 8; row < n; row += kTailBlock / 8) {
+        double acc = 0.0;
+        for (int j = lane; j < n; j += 8) acc += V.dense[row * n + j] * rc[j];
+        acc = group_sum<8>(acc);
+        if (lane == 0) {
+            zc[row] = (T)acc;
+            if (!task.pad) V.z[row] = (T)acc;
+        }
+    }
+    if (!task.pad) return;
+    __syncthreads();
+    if (Vf.ap_lanes == 4) tail_up<T, 4>(Vf, tl, zc);
+    else if (Vf.ap_lanes == 8) tail_up<T, 8>(Vf, tl, zc);
+    else tail_up<T, 16>(Vf, tl, zc);
+}
+
+// z = w' + omega B^-1 (t - alpha (A P) z_{l+1}),  w' = w + alpha P z_{l+1} (level 0: full
+// rows only); A P in FP32 when the view holds it so (APf).
+template <int NF, int MODE, typename T>
+__device__ __forceinline__ void post_rows(const AmgView<T>& V, const BlockTask& task, int which) {
+    struct Pre {
+        T w, z, t[NF], brow[NF];
+    };
+    const int N = V.A.N;
+    const T om = (T)V.omega, al = (T)V.alpha;
+    auto xat = [&](long long j, T (&xv)[NF]) { at_node<NF>(V.next_z.get(), j, xv); };
+    auto prod = [&](long long c, int k0, int step, T (&acc)[NF]) {
+        if (V.APf.vals) slice_part<NF, (MODE & ELL_STREAM) != 0>(V.APf, c, k0, step, xat, acc);
+        else slice_part<NF, (MODE & ELL_STREAM) != 0>(V.AP, c, k0, step, xat, acc);
+    };
+    auto pre = [&](long long i, int f) {
+        Pre o;
+        const int I = V.fine_agg[i];
+        const bool full = I >= 0 && (!V.mask || row_full_flags(V.flags[i], f, NF - 1));
+        o.w = V.w[i * NF + f];
+        at_node<NF>((const T*)V.t, i, o.t);
+        load_block_row<NF>((const T*)V.binv, N, f, i, o.brow);
+        const T z = V.next_z[(long long)max(I, 0) * NF + f];
+        o.z = full ? z : T(0);
+        return o;
+    };
+    auto fin = [&](long long i, int f, const T (&y)[NF], const Pre& o, int h) {
+        if (h) return;
+        T d[NF];
+#pragma unroll
+        for (int t = 0; t < NF; ++t) d[t] = o.t[t] - al * y[t];
+        const T out = (o.w + al * o.z) + om * block_row<NF>(o.brow, d);
+        if (V.level == 0) V.out0[which][i * NF + f] = (double)out;
+        else V.z[i * NF + f] = out;
+    };
+    slice_products<NF, MODE, T>(task, V.AP.nsl, N, prod, pre, fin);
+}
+
+template <typename T, bool STREAM>
 __global__ __launch_bounds__(kBlock) void k_amg_post(const AmgView<T>* __restrict__ views,
                                                      const BlockTask* __restrict__ tasks, int which) {
     const BlockTask task = tasks[blockIdx.x];
     if (task.case_id < 0) return;
     const AmgView<T>& V = views[task.case_id];
     if (*V.done_flag) return;
-    if (V.A.nf == 4) post_ell<4>(V, task, which);
-    else post_ell<3>(V, task, which);
+    PFEM_NF_MODE(post_rows, STREAM, V.A.nf, V.split, V, task, which);
 }
 
 // ---- launchers ---------------------------------------------------------------------------
@@ -476,35 +583,42 @@ void launch_amg_dense(const AmgView<T>* v, const BlockTask* t, int nt, hipStream
     k_amg_dense<T><<<nt, kBlock, 0, s>>>(v, t);
 }
 template <typename T>
-void launch_amg_res(const AmgView<T>* v, const BlockTask* t, int nt, int which, hipStream_t s) {
-    k_amg_res<T><<<nt, kBlock, 0, s>>>(v, t, which);
+void launch_amg_res(const AmgView<T>* v, const BlockTask* t, int nt, int which, bool stream, hipStream_t s) {
+    if (stream) k_amg_res<T, true><<<nt, kBlock, 0, s>>>(v, t, which);
+    else k_amg_res<T, false><<<nt, kBlock, 0, s>>>(v, t, which);
 }
 template <typename T>
 void launch_amg_restrict(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t s) {
     k_amg_restrict<T><<<nt, kBlock, 0, s>>>(v, t);
 }
 template <typename T>
-void launch_amg_coarsest(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t s) {
-    k_amg_coarsest<T><<<nt, kBlock, 0, s>>>(v, t);
+void launch_amg_rr(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t s) {
+    k_amg_rr<T><<<nt, kBlock, 0, s>>>(v, t);
+}
+template <typename T>
+void launch_amg_tail(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t s) {
+    k_amg_tail<T><<<nt, kTailBlock, 0, s>>>(v, t);
 }
 template <typename T>
 void launch_amg_ap(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t s) {
     k_amg_ap<T><<<nt, kBlock, 0, s>>>(v, t);
 }
 template <typename T>
-void launch_amg_post(const AmgView<T>* v, const BlockTask* t, int nt, int which, hipStream_t s) {
-    k_amg_post<T><<<nt, kBlock, 0, s>>>(v, t, which);
+void launch_amg_post(const AmgView<T>* v, const BlockTask* t, int nt, int which, bool stream, hipStream_t s) {
+    if (stream) k_amg_post<T, true><<<nt, kBlock, 0, s>>>(v, t, which);
+    else k_amg_post<T, false><<<nt, kBlock, 0, s>>>(v, t, which);
 }
 
 #define PFEM_AMG_INSTANTIATE(T)                                                                    \
     template void launch_amg_galerkin<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);   \
     template void launch_amg_bjac<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);       \
     template void launch_amg_dense<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);      \
-    template void launch_amg_res<T>(const AmgView<T>*, const BlockTask*, int, int, hipStream_t);   \
+    template void launch_amg_res<T>(const AmgView<T>*, const BlockTask*, int, int, bool, hipStream_t); \
     template void launch_amg_restrict<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);   \
-    template void launch_amg_coarsest<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);   \
+    template void launch_amg_rr<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);         \
+    template void launch_amg_tail<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);       \
     template void launch_amg_ap<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);         \
-    template void launch_amg_post<T>(const AmgView<T>*, const BlockTask*, int, int, hipStream_t);
+    template void launch_amg_post<T>(const AmgView<T>*, const BlockTask*, int, int, bool, hipStream_t);
 PFEM_AMG_INSTANTIATE(double)
 PFEM_AMG_INSTANTIATE(float)
 

@@ -1,9 +1,9 @@
 // SpMV over the sliced ELL copy of a PSPG system (EllMat): lane r of a wavefront computes
 // the NF rows of node 64 c + r of slice c.  Each rank k is one column node j (one index
 // load, NF gathers of x) and NF*NF value loads, each 64 consecutive doubles per wavefront.
-// The values are loaded non-temporally: they are read once per launch, and without the hint
-// they evict the x entries and the results from the caches (measured on gfx950, 516 MB
-// matrix: 98.7 -> 90.0 us per launch; 2D 900k nodes: 104 -> 94 us).
+// Of matrices larger than the caches the values are loaded non-temporally (ELL_STREAM): they are
+// read once per launch, and without the hint they evict the x entries and the results from the
+// caches (516 MB matrix: 98.7 -> 90.0 us per launch; 2D 900k nodes: 104 -> 94 us).
 #pragma once
 
 #include "common.hpp"
@@ -15,7 +15,7 @@ namespace pfem {
 // acc[s] = (A x) of row (64 c + lane, s) over the ranks k0, k0 + step, ... of slice c, with values
 // of type VT and vectors and sums of type XT; xat(j, xv) gives the NF entries of x at node j.
 // Lanes past the last node compute values that the callers drop.
-template <int NF, typename VT, typename XT, class X>
+template <int NF, bool STREAM, typename VT, typename XT, class X>
 __device__ __forceinline__ void slice_part(const EllMatT<VT>& E, long long c, int k0, int step, X&& xat,
                                            XT (&acc)[NF]) {
     const int lane = threadIdx.x & (kEllSlice - 1);
@@ -33,7 +33,10 @@ __device__ __forceinline__ void slice_part(const EllMatT<VT>& E, long long c, in
         for (int s = 0; s < NF; ++s)
 #pragma unroll
             for (int t = 0; t < NF; ++t)
-                a[s][t] = (XT)ld_stream(vb + ((long long)k * NF * NF + s * NF + t) * kEllSlice);
+            {
+                const VT* q = vb + ((long long)k * NF * NF + s * NF + t) * kEllSlice;
+                a[s][t] = (XT)(STREAM ? ld_stream(q) : *q);
+            }
         XT xv[NF];
         xat(j, xv);
 #pragma unroll
@@ -55,14 +58,14 @@ __device__ __forceinline__ void at_node(const T* __restrict__ x, long long j, T 
     for (int t = 0; t < NF; ++t) xv[t] = x[j * NF + t];
 }
 
-// y[f] without dynamic register indexing.
+// y[f] without dynamic register indexing (the values are pinned in registers: a selected address
+// would put the array into LDS).
 template <int NF, typename T>
 __device__ __forceinline__ T at_field(const T (&y)[NF], int f) {
-    T r = y[0];
-#pragma unroll
-    for (int s = 1; s < NF; ++s)
-        if (s == f) r = y[s];
-    return r;
+    T a = y[0], b = y[1], c = y[2], d = y[NF - 1];
+    asm volatile("" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
+    const T lo = (f & 1) ? b : a, hi = (f & 1) ? d : c;
+    return (f & 2) ? hi : lo;
 }
 
 // Row f of B^-1 times the node's NF values.
@@ -85,15 +88,15 @@ __device__ __forceinline__ void load_block_row(const T* __restrict__ binv, long 
 // pre(i, f) loads what row f of node i < rows needs besides (issued before any store), and
 // fin(i, f, y, pre's result, h) finishes that row from the node's NF products y, h = 0 and then 1
 // (a result per pass: the stores of one lane's fields to one vector then merge).
-// SPLIT: the four wavefronts share a slice, add their parts through LDS in order and finish the
+// ELL_SPLIT: the four wavefronts share a slice, add their parts through LDS in order and finish the
 // slice's rows in the order of node-blocked vectors (thread e: node e / NF, field e % NF); else
 // each wavefront takes whole slices, one lane per node.
-template <int NF, bool SPLIT, typename T, class PR, class PRE, class FI>
+template <int NF, int MODE, typename T, class PR, class PRE, class FI>
 __device__ __forceinline__ void slice_products(const BlockTask& task, int nsl, long long rows, PR&& prod, PRE&& pre,
                                                FI&& fin) {
     const Seg sg = xcd_segment(task, nsl);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if constexpr (SPLIT) {
+    if constexpr ((MODE & ELL_SPLIT) != 0) {
         __shared__ T red[kWaves][NF][kEllSlice];
         const int n = threadIdx.x / NF, f = threadIdx.x - n * NF;
         for (int l = sg.lb; l < sg.ns; l += sg.cnt) {
@@ -141,11 +144,12 @@ __device__ __forceinline__ void slice_products(const BlockTask& task, int nsl, l
     }
 }
 
-// Calls BODY<NF, SPLIT> for a view's fields and split.
-#define PFEM_NF_SPLIT(BODY, nf, split, ...)                                          \
-    do {                                                                             \
-        if ((nf) == 4) (split) ? BODY<4, true>(__VA_ARGS__) : BODY<4, false>(__VA_ARGS__); \
-        else (split) ? BODY<3, true>(__VA_ARGS__) : BODY<3, false>(__VA_ARGS__);     \
+// Calls BODY<NF, MODE> for a view's fields and split and the launch's STREAM.
+#define PFEM_NF_MODE(BODY, STREAM, nf, split, ...)                                                      \
+    do {                                                                                                \
+        constexpr int kWhole = (STREAM) ? ELL_STREAM : 0;                                               \
+        if ((nf) == 4) (split) ? BODY<4, kWhole | ELL_SPLIT>(__VA_ARGS__) : BODY<4, kWhole>(__VA_ARGS__); \
+        else (split) ? BODY<3, kWhole | ELL_SPLIT>(__VA_ARGS__) : BODY<3, kWhole>(__VA_ARGS__);         \
     } while (0)
 
 }  // namespace pfem

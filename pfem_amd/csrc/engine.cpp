@@ -136,12 +136,18 @@ int row_blocks(long long n, int nsl) {
 }
 
 // A workgroup's wavefronts share a slice while all the workgroups run at once (768: three per CU;
-// their registers allow four).  Measured per iteration, shared / one wavefront per slice: 188
-// slices (12k nodes, 3D FP64) 31 / 46 us, 16 (1k, 2D) 16 / 19, 313 (20k, 2D, multigrid's part) 25 /
-// 33, 750 (48k, 3D FP64) 76 / 75, 1,125 (72k, 3D FP32) 67 / 54, 4,110 (263k, 3D FP64) 260 / 228.
-bool kry_split(int nsl) { return nsl <= 768; }
+// their registers allow four).  Measured per BiCGSTAB iteration, shared / one wavefront per slice:
+// 16 slices (1k nodes, 2D) 16 / 19 us, 188 (12k, 3D FP64) 31 / 46, 750 (48k, 3D FP64) 76 / 75, 1,125
+// (72k, 3D FP32) 67 / 54, 4,110 (263k, 3D FP64) 260 / 228.
+bool split_slices(int nsl) { return nsl <= 768; }
+
+// While a launch's matrices leave half of the 256 MB memory-side cache free they are read with
+// plain loads: the non-temporal ones pass it by.  Product with plain / non-temporal loads: 12k nodes
+// (3D FP64, 24 MB) 9.4 / 12.2 us, 72k FP32 (69 MB) 15.2 / 18.8, 60k FP64 (115 MB) 19.9 / 22.6; at
+// 110k (211 MB) 40.7 / 40.6, with the multigrid's other kernels 15 % slower for want of the cache.
+bool stream_values(long long value_bytes) { return value_bytes > (160LL << 20); }
 int kry_blocks(int nsl) {
-    return kry_split(nsl) ? std::max(1, nsl) : row_blocks(1, nsl);
+    return split_slices(nsl) ? std::max(1, nsl) : row_blocks(1, nsl);
 }
 
 // lanes per field of the node-block SpMV: the node-graph degree (incl. the node itself)
@@ -576,7 +582,7 @@ void Engine::Impl::load_views(Req* r) {
         k.nodes = N;
         k.nf = dim + 1;
         k.nblk = kry_blocks(P.ell_nsl);
-        k.split = kry_split(P.ell_nsl);
+        k.split = split_slices(P.ell_nsl);
         k.binv = w.binv;
         k.b = w.b;
         k.x = w.x;
@@ -615,7 +621,7 @@ void Engine::Impl::load_views(Req* r) {
             f.nodes = N;
             f.nf = dim + 1;
             f.nblk = kry_blocks(P.ell_nsl);
-            f.split = kry_split(P.ell_nsl);
+            f.split = split_slices(P.ell_nsl);
             f.E = ell_mat<float>(P, dim, w.vals32_ell);  // the inner solve's SpMVs run over the FP32 ELL copy
             f.binv = w.binv32;
             f.b = u;
@@ -733,6 +739,7 @@ void Engine::Impl::load_amg(pfem_case* c, int slot, const KrylovView<double>& k,
         V.omega = std::min(amg_omega, c->amg_omega_cap);
         V.alpha = amg_alpha;
         V.done_flag = &ds->k[0].done;
+        V.split = split_slices(((l == 0 ? c->N : H.lev[l].N) + kEllSlice - 1) / kEllSlice);
         if (l == 0) {
             V.A = A0;
             V.binv = binv0;
@@ -1045,6 +1052,7 @@ void Engine::tick(std::vector<Req*>& done) {
 
     // ---- work tables ------------------------------------------------------------------
     std::vector<BlockTask> tab[T_NTAB];
+    long long value_bytes = 0;            // matrices the tick's products read
     int wc_cap[2][2] = {{0, 0}, {0, 0}};  // most nodes a WC tile stages, by state type and dimension
     for (Req* r : inflight_) {
         pfem_case* c = r->c;
@@ -1064,6 +1072,9 @@ void Engine::tick(std::vector<Req*>& done) {
         if (op & OP_IRU) append_rows(tab[T_IRU], sl, c->n, c->pat.ell_nsl);
         if (op & OP_IRR) append_rows(tab[T_IRR + li], sl, c->n, c->pat.ell_nsl);
         const int nk = kry_blocks(c->pat.ell_nsl);
+        if (op & (OP_K64_INIT | OP_K64_RUN | OP_K32_INIT | OP_K32_RUN))
+            value_bytes += c->pat.ell_ranks * kEllSlice * (c->dim + 1) * (c->dim + 1) *
+                           ((op & (OP_K64_INIT | OP_K64_RUN)) ? 8LL : 4LL);
         if (op & OP_K64_RUN)
             for (int b = 0; b < nk; ++b) tab[T_K64].push_back(BlockTask{sl, b, nk, 0});
         if (op & OP_K32_RUN)
@@ -1089,14 +1100,18 @@ void Engine::tick(std::vector<Req*>& done) {
                 }
             }
             if (op & OP_K64_RUN) {
-                for (int l = 0; l + 1 < H.levels; ++l) {
-                    const int Nl = l == 0 ? c->N : H.lev[l].N;
-                    const int lanes = l == 0 ? c->lanes : H.lev[l].lanes;
-                    append(A[A_VN + l], base + l, Nl, kElemCap);
-                    if (l > 0) append(A[A_VS + l], base + l, (long long)Nl * lanes, kElemCap);
-                    append(A[A_VR + l], base + l, (long long)H.lev[l + 1].N * kRestrictLanes, kElemCap);
+                const int last = H.levels - 1;
+                const int nf = c->dim + 1;
+                const bool tail = last >= 2 && H.lev[last - 1].N <= kAmgTailNodes &&
+                                  nf * nf * H.lev[last - 1].graph_nnz <= kAmgTailValues;
+                for (int l = 0; l < (tail ? last - 1 : last); ++l) {
+                    const int Nl = l == 0 ? c->N : H.lev[l].N, nsl = (Nl + kEllSlice - 1) / kEllSlice;
+                    const int nb = kry_blocks(nsl);
+                    for (int b = 0; b < nb; ++b) A[A_VN + l].push_back(BlockTask{base + l, b, nb, 0});
+                    if (l > 0) append(A[A_VS + l], base + l, (long long)H.lev[l + 1].N * kBlock, kElemCap);
+                    else append(A[A_VR + l], base + l, (long long)H.lev[l + 1].N * kRestrictLanes, kElemCap);
                 }
-                A[A_VC].push_back(BlockTask{base + H.levels - 1, 0, 1, 0});
+                A[A_VC].push_back(BlockTask{base + last, 0, 1, tail ? 1 : 0});
             }
         }
         const int wi = c->d.wc_state == PFEM_STATE_FP32 ? 1 : 0;
@@ -1176,8 +1191,9 @@ void Engine::tick(std::vector<Req*>& done) {
         if (NT(T_IRR + li)) launch_ir_residual(kLanes[li], vref, T(T_IRR + li), NT(T_IRR + li), s);
     const KrylovView<double>* vk64 = I.d_k64.as<KrylovView<double>>();
     const KrylovView<float>* vk32 = I.d_k32.as<KrylovView<float>>();
-    if (NT(T_F64)) launch_kry_init<double>(vk64, T(T_K64), NT(T_K64), T(T_F64), NT(T_F64), I.par ^ 1, s);
-    if (NT(T_F32)) launch_kry_init<float>(vk32, T(T_K32), NT(T_K32), T(T_F32), NT(T_F32), I.par ^ 1, s);
+    const bool stream = stream_values(value_bytes);
+    if (NT(T_F64)) launch_kry_init<double>(vk64, T(T_K64), NT(T_K64), T(T_F64), NT(T_F64), I.par ^ 1, stream, s);
+    if (NT(T_F32)) launch_kry_init<float>(vk32, T(T_K32), NT(T_K32), T(T_F32), NT(T_F32), I.par ^ 1, stream, s);
     // live SpMV timing: one request iterating alone
     int prof_w = -1, prof_before = 0;
     if (I.prof && nrun == 1) {
@@ -1189,21 +1205,19 @@ void Engine::tick(std::vector<Req*>& done) {
             }
     }
     // multigrid V-cycle of the cases that have a hierarchy: which = 0 (ph = M^-1 p) or 1 (sh = M^-1 s).
-    // Level 0's residual and every level's post-smoothing run one lane per node over ELL
-    // slices (table A_VN: N_l / kBlock workgroups per case); the residual of the coarser
-    // levels runs `lanes` lanes per node (A_VS).
+    // Level 0's residual and every level's post-smoothing walk ELL slices (table A_VN); residual
+    // and restriction of the coarser levels take a workgroup per aggregate (A_VS).
     auto vcycle_type = [&](auto* v, int TA, int which) {
         for (int l = 0; l < kAmgMaxLevels; ++l) {
-            if (!NT(TA + A_VN + l)) break;
-            const int tr = TA + (l == 0 ? A_VN : A_VS) + l;
-            // the pre-smoothing of levels >= 1 is part of the restriction from the finer level,
-            // that of level 0 part of BiCGSTAB's U and S (KrylovView::mg_w0)
-            launch_amg_res(v, T(tr), NT(tr), which, s);
-            launch_amg_restrict(v, T(TA + A_VR + l), NT(TA + A_VR + l), s);
+            if (NT(TA + A_VR + l)) {
+                launch_amg_res(v, T(TA + A_VN + l), NT(TA + A_VN + l), which, stream, s);
+                launch_amg_restrict(v, T(TA + A_VR + l), NT(TA + A_VR + l), s);
+            }
+            if (NT(TA + A_VS + l)) launch_amg_rr(v, T(TA + A_VS + l), NT(TA + A_VS + l), s);
         }
-        if (NT(TA + A_VC)) launch_amg_coarsest(v, T(TA + A_VC), NT(TA + A_VC), s);
+        if (NT(TA + A_VC)) launch_amg_tail(v, T(TA + A_VC), NT(TA + A_VC), s);
         for (int l = kAmgMaxLevels - 1; l >= 0; --l)
-            if (NT(TA + A_VN + l)) launch_amg_post(v, T(TA + A_VN + l), NT(TA + A_VN + l), which, s);
+            if (NT(TA + A_VN + l)) launch_amg_post(v, T(TA + A_VN + l), NT(TA + A_VN + l), which, stream, s);
     };
     auto vcycle = [&](int which) {
         vcycle_type(vamg64, T_AMG, which);
@@ -1215,10 +1229,10 @@ void Engine::tick(std::vector<Req*>& done) {
             const int p = (I.par + it) & 1;
             for (int phase = 0; phase < 4; ++phase) {
                 if (NT(T_K64) && (phase != 2 || multigrid))  // S belongs to the multigrid cases
-                    launch_kry_phase<double>(phase, vk64, T(T_K64), NT(T_K64), p, s,
+                    launch_kry_phase<double>(phase, vk64, T(T_K64), NT(T_K64), p, stream, s,
                                              (phase == 1 && prof_w == 0) ? I.pev + 2 * it : nullptr);
                 if (NT(T_K32) && phase != 2)
-                    launch_kry_phase<float>(phase, vk32, T(T_K32), NT(T_K32), p, s,
+                    launch_kry_phase<float>(phase, vk32, T(T_K32), NT(T_K32), p, stream, s,
                                             (phase == 1 && prof_w == 1) ? I.pev + 2 * it : nullptr);
                 if (phase == 0) vcycle(0);
                 if (phase == 2) vcycle(1);
@@ -1227,12 +1241,13 @@ void Engine::tick(std::vector<Req*>& done) {
     };
     bool replayed = false;
     if (I.graphs && chunk > 0 && prof_w < 0) {
-        // everything the chunk's launches capture: its length and parity, the base addresses of
+        // everything the chunk's launches capture: its length, parity and kind of loads, the base addresses of
         // the tables and views, and the tables' layout and contents
         std::vector<long long> key;
         key.reserve(16 + T_NTAB + 4 * total);
         key.push_back(chunk);
         key.push_back(I.par);
+        key.push_back(stream);
         for (const void* p : {I.d_tab.p, I.d_k64.p, I.d_k32.p, I.d_amg64.p, I.d_amg32.p})
             key.push_back((long long)(uintptr_t)p);
         for (int t = 0; t <= T_NTAB; ++t) key.push_back((long long)off[t]);

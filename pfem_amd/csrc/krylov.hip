@@ -94,7 +94,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv(NodeMat<T> A, const T* __restri
 }
 
 // (Re)start: r = b - A x (or b when x_zero), rh = r.
-template <int NF, bool SPLIT, typename T>
+template <int NF, int MODE, typename T>
 __device__ __forceinline__ void init_body(const KrylovView<T>& V, const BlockTask& task, double (&part)[3]) {
     const T* __restrict__ x = V.x;
     const long long N = V.nodes;
@@ -103,7 +103,7 @@ __device__ __forceinline__ void init_body(const KrylovView<T>& V, const BlockTas
 #pragma unroll
             for (int t = 0; t < NF; ++t) acc[t] = T(0);
         } else {
-            slice_part<NF>(V.E, c, k0, step, [&](long long j, T (&xv)[NF]) { at_fields<NF>(x, N, j, xv); }, acc);
+            slice_part<NF, (MODE & ELL_STREAM) != 0>(V.E, c, k0, step, [&](long long j, T (&xv)[NF]) { at_fields<NF>(x, N, j, xv); }, acc);
         }
     };
     auto pre = [&](long long i, int f) { return V.b[i + f * N]; };
@@ -117,10 +117,10 @@ __device__ __forceinline__ void init_body(const KrylovView<T>& V, const BlockTas
         part[1] += (double)r * (double)r;
         part[2] += (double)bi * (double)bi;
     };
-    slice_products<NF, SPLIT, T>(task, V.E.nsl, N, prod, pre, fin);
+    slice_products<NF, MODE, T>(task, V.E.nsl, N, prod, pre, fin);
 }
 
-template <typename T>
+template <typename T, bool STREAM>
 __global__ __launch_bounds__(kBlock) void k_kry_init(const KrylovView<T>* __restrict__ views,
                                                      const BlockTask* __restrict__ tasks) {
     const BlockTask task = tasks[blockIdx.x];
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(kBlock) void k_kry_init(const KrylovView<T>* __rest
     const KrylovView<T>& V = views[task.case_id];
     if (!V.sc->req_init) return;
     double part[3] = {0.0, 0.0, 0.0};
-    PFEM_NF_SPLIT(init_body, V.nf, V.split, V, task, part);
+    PFEM_NF_MODE(init_body, STREAM, V.nf, V.split, V, task, part);
     constexpr int slots[3] = {P_RHR, P_RR, P_BB};
     write_partials<3>(part, V.partials, task.block, slots);
 }
@@ -299,14 +299,14 @@ __global__ __launch_bounds__(kBlock) void k_kry_update(const KrylovView<T>* __re
 }
 
 // V: v = A ph (and vhat = B^-1 v); part = {(rh, v)}.
-template <int NF, bool SPLIT, bool AMG, typename T>
+template <int NF, int MODE, bool AMG, typename T>
 __device__ __forceinline__ void v_rows(const KrylovView<T>& V, const BlockTask& task, double (&part)[1]) {
     struct Pre {
         T rh, brow[NF];
     };
     const T* __restrict__ x = V.ph;
     auto prod = [&](long long c, int k0, int step, T (&acc)[NF]) {
-        slice_part<NF>(V.E, c, k0, step, [&](long long j, T (&xv)[NF]) { at_node<NF>(x, j, xv); }, acc);
+        slice_part<NF, (MODE & ELL_STREAM) != 0>(V.E, c, k0, step, [&](long long j, T (&xv)[NF]) { at_node<NF>(x, j, xv); }, acc);
     };
     auto pre = [&](long long i, int f) {
         Pre o;
@@ -323,16 +323,16 @@ __device__ __forceinline__ void v_rows(const KrylovView<T>& V, const BlockTask& 
         V.v[i * NF + f] = v;
         part[0] += (double)o.rh * (double)v;
     };
-    slice_products<NF, SPLIT, T>(task, V.E.nsl, V.nodes, prod, pre, fin);
+    slice_products<NF, MODE, T>(task, V.E.nsl, V.nodes, prod, pre, fin);
 }
 
-template <int NF, bool SPLIT, typename T>
+template <int NF, int MODE, typename T>
 __device__ __forceinline__ void v_body(const KrylovView<T>& V, const BlockTask& task, double (&part)[1]) {
-    if (V.amg) v_rows<NF, SPLIT, true>(V, task, part);
-    else v_rows<NF, SPLIT, false>(V, task, part);
+    if (V.amg) v_rows<NF, MODE, true>(V, task, part);
+    else v_rows<NF, MODE, false>(V, task, part);
 }
 
-template <typename T>
+template <typename T, bool STREAM>
 __global__ __launch_bounds__(kBlock) void k_kry_v(const KrylovView<T>* __restrict__ views,
                                                   const BlockTask* __restrict__ tasks, int par) {
     const BlockTask task = tasks[blockIdx.x];
@@ -341,7 +341,7 @@ __global__ __launch_bounds__(kBlock) void k_kry_v(const KrylovView<T>* __restric
     KScal& S = *V.sc;
     if (S.done) return;
     double part[1] = {0.0};
-    PFEM_NF_SPLIT(v_body, V.nf, V.split, V, task, part);
+    PFEM_NF_MODE(v_body, STREAM, V.nf, V.split, V, task, part);
     constexpr int slots[1] = {P_RV};
     write_partials<1>(part, V.partials, task.block, slots);
 }
@@ -419,7 +419,7 @@ __global__ __launch_bounds__(kBlock) void k_kry_s(const KrylovView<T>* __restric
 }
 
 // T: part = {(t, s), (t, t), (rh, t)} and, with block Jacobi, {(s, s), (rh, s)}.
-template <int NF, bool SPLIT, bool AMG, typename T>
+template <int NF, int MODE, bool AMG, typename T>
 __device__ __forceinline__ void t_rows(const KrylovView<T>& V, const BlockTask& task, double alpha, double (&part)[5]) {
     struct Pre {
         T rh, s, r, v;
@@ -437,7 +437,7 @@ __device__ __forceinline__ void t_rows(const KrylovView<T>& V, const BlockTask& 
                 for (int t = 0; t < NF; ++t) xv[t] -= a * hv[t];
             }
         };
-        slice_part<NF>(V.E, c, k0, step, xat, acc);
+        slice_part<NF, (MODE & ELL_STREAM) != 0>(V.E, c, k0, step, xat, acc);
     };
     auto pre = [&](long long i, int f) {
         const long long q = i * NF + f;
@@ -463,16 +463,16 @@ __device__ __forceinline__ void t_rows(const KrylovView<T>& V, const BlockTask& 
             part[4] += (double)o.rh * (double)s;
         }
     };
-    slice_products<NF, SPLIT, T>(task, V.E.nsl, V.nodes, prod, pre, fin);
+    slice_products<NF, MODE, T>(task, V.E.nsl, V.nodes, prod, pre, fin);
 }
 
-template <int NF, bool SPLIT, typename T>
+template <int NF, int MODE, typename T>
 __device__ __forceinline__ void t_body(const KrylovView<T>& V, const BlockTask& task, double alpha, double (&part)[5]) {
-    if (V.amg) t_rows<NF, SPLIT, true>(V, task, alpha, part);
-    else t_rows<NF, SPLIT, false>(V, task, alpha, part);
+    if (V.amg) t_rows<NF, MODE, true>(V, task, alpha, part);
+    else t_rows<NF, MODE, false>(V, task, alpha, part);
 }
 
-template <typename T>
+template <typename T, bool STREAM>
 __global__ __launch_bounds__(kBlock) void k_kry_t(const KrylovView<T>* __restrict__ views,
                                                   const BlockTask* __restrict__ tasks, int par) {
     const BlockTask task = tasks[blockIdx.x];
@@ -481,7 +481,7 @@ __global__ __launch_bounds__(kBlock) void k_kry_t(const KrylovView<T>* __restric
     if (V.sc->done) return;
     double part[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, alpha = 0.0;
     if (!V.amg && !step_alpha(V, task, par, alpha)) return;
-    PFEM_NF_SPLIT(t_body, V.nf, V.split, V, task, alpha, part);
+    PFEM_NF_MODE(t_body, STREAM, V.nf, V.split, V, task, alpha, part);
     if (V.amg) {  // S has written the other two
         double p3[3] = {part[0], part[1], part[2]};
         constexpr int slots[3] = {P_TS, P_TT, P_RHT};
@@ -543,27 +543,36 @@ __global__ __launch_bounds__(kBlock) void k_ir_update(const RefineView* __restri
 
 template <typename T>
 void launch_kry_init(const KrylovView<T>* v, const BlockTask* t, int nt, const BlockTask* ids, int nids, int par,
-                     hipStream_t s) {
-    k_kry_init<T><<<nt, kBlock, 0, s>>>(v, t);
+                     bool stream, hipStream_t s) {
+    if (stream) k_kry_init<T, true><<<nt, kBlock, 0, s>>>(v, t);
+    else k_kry_init<T, false><<<nt, kBlock, 0, s>>>(v, t);
     k_kry_init_fin<T><<<nids < 1024 ? nids : 1024, kBlock, 0, s>>>(v, ids, nids, par);
 }
 
 // One kernel of an iteration (phase 0 U, 1 V, 2 S, 3 T) with parity par, so that a
-// preconditioner's launches can sit between them; ev (optional) brackets V.
-template <typename T>
-void launch_kry_phase(int phase, const KrylovView<T>* v, const BlockTask* t, int nt, int par, hipStream_t s,
+// preconditioner's launches can sit between them; stream: non-temporal value loads; ev
+// (optional) brackets V.
+template <typename T, bool STREAM>
+static void kry_phase(int phase, const KrylovView<T>* v, const BlockTask* t, int nt, int par, hipStream_t s,
                       hipEvent_t* ev) {
     switch (phase) {
         case 0: k_kry_update<T><<<nt, kBlock, 0, s>>>(v, t, par); break;
         case 1:
             // timed: the events ride on the dispatch itself (start and end of the kernel,
             // as a profiler sees them), not as separate packets around it
-            if (ev) hipExtLaunchKernelGGL(k_kry_v<T>, dim3(nt), dim3(kBlock), 0, s, ev[0], ev[1], 0, v, t, par);
-            else k_kry_v<T><<<nt, kBlock, 0, s>>>(v, t, par);
+            if (ev) hipExtLaunchKernelGGL((k_kry_v<T, STREAM>), dim3(nt), dim3(kBlock), 0, s, ev[0], ev[1], 0, v, t, par);
+            else k_kry_v<T, STREAM><<<nt, kBlock, 0, s>>>(v, t, par);
             break;
         case 2: k_kry_s<T><<<nt, kBlock, 0, s>>>(v, t, par); break;
-        default: k_kry_t<T><<<nt, kBlock, 0, s>>>(v, t, par); break;
+        default: k_kry_t<T, STREAM><<<nt, kBlock, 0, s>>>(v, t, par); break;
     }
+}
+
+template <typename T>
+void launch_kry_phase(int phase, const KrylovView<T>* v, const BlockTask* t, int nt, int par, bool stream,
+                      hipStream_t s, hipEvent_t* ev) {
+    if (stream) kry_phase<T, true>(phase, v, t, nt, par, s, ev);
+    else kry_phase<T, false>(phase, v, t, nt, par, s, ev);
 }
 
 // y = A x over the sliced ELL copy (one wavefront per 64-node slice), the SpMV the BiCGSTAB
@@ -574,7 +583,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_ell(const EllMatT<double> E, co
     const int lane = threadIdx.x & (kEllSlice - 1);
     for (long long c = (long long)blockIdx.x * kWaves + (threadIdx.x >> 6); c < E.nsl; c += (long long)gridDim.x * kWaves) {
         double r[NF];
-        slice_part<NF>(E, c, 0, 1, [&](long long j, double (&xv)[NF]) { at_fields<NF>(x, E.N, j, xv); }, r);
+        slice_part<NF, true>(E, c, 0, 1, [&](long long j, double (&xv)[NF]) { at_fields<NF>(x, E.N, j, xv); }, r);
         const long long i = c * kEllSlice + lane;
         if (i < E.N)
 #pragma unroll
@@ -601,12 +610,12 @@ void launch_ir_update(const RefineView* v, const BlockTask* t, int nt, hipStream
 }
 
 template void launch_kry_init<double>(const KrylovView<double>*, const BlockTask*, int, const BlockTask*, int, int,
-                                      hipStream_t);
+                                      bool, hipStream_t);
 template void launch_kry_init<float>(const KrylovView<float>*, const BlockTask*, int, const BlockTask*, int, int,
-                                     hipStream_t);
-template void launch_kry_phase<double>(int, const KrylovView<double>*, const BlockTask*, int, int, hipStream_t,
+                                     bool, hipStream_t);
+template void launch_kry_phase<double>(int, const KrylovView<double>*, const BlockTask*, int, int, bool, hipStream_t,
                                        hipEvent_t*);
-template void launch_kry_phase<float>(int, const KrylovView<float>*, const BlockTask*, int, int, hipStream_t,
+template void launch_kry_phase<float>(int, const KrylovView<float>*, const BlockTask*, int, int, bool, hipStream_t,
                                       hipEvent_t*);
 template void launch_spmv<double>(int, const NodeMat<double>&, const double*, double*, int, hipStream_t);
 template void launch_spmv<float>(int, const NodeMat<float>&, const float*, float*, int, hipStream_t);

@@ -13,9 +13,9 @@ void launch_pspg_bc(const PspgView* views, const BlockTask* tasks, int ntasks, h
 // ids: the cases (case_id of each entry) whose KScal::req_init is set, nids of them
 template <typename T>
 void launch_kry_init(const KrylovView<T>* v, const BlockTask* t, int nt, const BlockTask* ids, int nids, int par,
-                     hipStream_t s);
+                     bool stream, hipStream_t s);
 template <typename T>
-void launch_kry_phase(int phase, const KrylovView<T>* v, const BlockTask* t, int nt, int par, hipStream_t s,
+void launch_kry_phase(int phase, const KrylovView<T>* v, const BlockTask* t, int nt, int par, bool stream, hipStream_t s,
                       hipEvent_t* ev = nullptr);
 template <typename T>
 void launch_spmv(int lanes, const NodeMat<T>& A, const T* x, T* y, int nblocks, hipStream_t s);
@@ -30,15 +30,17 @@ void launch_amg_bjac(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_
 template <typename T>
 void launch_amg_dense(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t s);
 template <typename T>
-void launch_amg_res(const AmgView<T>* v, const BlockTask* t, int nt, int which, hipStream_t s);
+void launch_amg_res(const AmgView<T>* v, const BlockTask* t, int nt, int which, bool stream, hipStream_t s);
 template <typename T>
 void launch_amg_restrict(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t s);
 template <typename T>
-void launch_amg_coarsest(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t s);
+void launch_amg_rr(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t s);
+template <typename T>
+void launch_amg_tail(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t s);
 template <typename T>
 void launch_amg_ap(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t s);
 template <typename T>
-void launch_amg_post(const AmgView<T>* v, const BlockTask* t, int nt, int which, hipStream_t s);
+void launch_amg_post(const AmgView<T>* v, const BlockTask* t, int nt, int which, bool stream, hipStream_t s);
 void launch_ir_residual(int lanes, const RefineView* v, const BlockTask* t, int nt, hipStream_t s);
 void launch_ir_update(const RefineView* v, const BlockTask* t, int nt, hipStream_t s);
 

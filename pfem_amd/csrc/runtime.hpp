@@ -200,10 +200,11 @@ int64_t now_ns();
 // workgroups per case of the row launches (Krylov, residual, refinement); nsl = the
 // case's ELL slices (0: none)
 int row_blocks(long long n, int nsl = 0);
-// whether the wavefronts of a workgroup share each ELL slice in a case's BiCGSTAB launches, and
-// the workgroups of those launches
-bool kry_split(int nsl);
+// whether the wavefronts of a workgroup share each ELL slice of a matrix, the workgroups of its
+// products' launches, and whether a launch over value_bytes of matrices loads them non-temporally
+bool split_slices(int nsl);
 int kry_blocks(int nsl);
+bool stream_values(long long value_bytes);
 int pick_lanes(double avg_deg);
 
 }  // namespace pfem

@@ -115,6 +115,10 @@ struct EllMatT {
 };
 using EllMat = EllMatT<double>;
 
+// Options of the products over such a matrix: a workgroup's four wavefronts share each slice (else
+// one wavefront per slice); non-temporal value loads.
+enum : int { ELL_SPLIT = 1, ELL_STREAM = 2 };
+
 // Scalars of one BiCGSTAB solve.  The per-iteration scalars live in two slots used
 // alternately (the host passes the slot parity of each iteration): a kernel only writes
 // the current slot and only reads the previous one or fields written by earlier kernels,
@@ -179,6 +183,10 @@ struct KrylovView {
 // kernels; T is the hierarchy's arithmetic type (FP64, or FP32 under FP64 BiCGSTAB: the
 // preconditioner only shapes the search directions, the solve converges on the FP64 system).
 constexpr int kAmgMaxDense = 88;  // coarsest-level unknowns inverted densely in LDS
+// The level above the coarsest is handled with it, in one workgroup, up to these sizes: the four
+// launches cost ~16 us, one workgroup 8 us on 60 nodes in 2D (4k values), 25 us on 250 (16k) and
+// 26-37 us on 100-200 nodes in 3D (50-90k values).
+constexpr int kAmgTailNodes = 128, kAmgTailValues = 6144;
 constexpr int kRestrictLanes = 8;  // lanes per aggregate of the restriction
 // Lanes per node in the PSPG assembly gathers (pair blocks, diagonal block and b).  Measured on
 // the 262k-node 3D dam break / a 100k-node 2D column, off-diagonal + diagonal kernels: 16 lanes
@@ -193,6 +201,7 @@ struct AmgView {
     Gp<const T> binv;         // block-Jacobi inverse, SoA [(nf*nf)][N]
     int level;
     int lanes;             // SpMV lanes per node on this level
+    int split, pad2;       // 1: the wavefronts of a workgroup share each slice (level 0 and A P products)
     int mask;              // level 0: transfers and Galerkin sums use full rows only
     Gp<const uint8_t> flags;  // level 0: the nodes' flags (the masks read them; 1 byte per node)
     int nc;                // coarsest level: unknowns of the dense inverse
