@@ -77,9 +77,10 @@ void setup_heat(pfem_case* c) {
     up(H.diag_pos, dpos.data(), sizeof(int) * dpos.size());
     const int nb = pfem::heat_blocks(N);
     H.vals.reserve(sizeof(double) * col.size());
-    for (pfem::DevBuf* b : {&H.b, &H.x, &H.r, &H.z, &H.p, &H.q, &H.dinv}) b->reserve(sizeof(double) * (size_t)N);
+    for (pfem::DevBuf* b : {&H.b, &H.x, &H.r, &H.z, &H.q, &H.dinv}) b->reserve(sizeof(double) * (size_t)N);
     H.erec.reserve(sizeof(double) * 16 * (size_t)E);
-    H.part.reserve(sizeof(double) * 5 * (size_t)nb);
+    H.part.reserve(sizeof(double) * (4 * (size_t)nb + pfem::kCgBlocks));
+    H.p.reserve(sizeof(double) * 2 * (size_t)N);
     H.scal.reserve(sizeof(double) * 2);
     H.T.reserve(sizeof(double) * (size_t)N);
     PFEM_HIP(hipMemsetAsync(H.T.p, 0, sizeof(double) * (size_t)N, c->stream));
@@ -100,6 +101,7 @@ pfem::HeatView heat_view(pfem_case* c, double dt) {
     V.E = c->E;
     V.F = H.F;
     V.nb = pfem::heat_blocks(c->N);
+    V.nq = pfem::cg_blocks(c->N, c->dim);
     V.conn = c->pat.conn.as<int>();
     V.flags = c->pat.flags.as<uint8_t>();
     V.pos = c->pos.as<double>();
@@ -152,12 +154,13 @@ void setup_frac(pfem_case* c) {
     F.mk.reserve(sizeof(double) * G * D * D);
     F.ms.reserve(sizeof(double) * G);
     F.lv.reserve(sizeof(double) * G);
-    for (DevBuf* b : {&F.dinv_mk, &F.dinv_m, &F.bv, &F.vt, &F.dv, &F.v_it, &F.v_itp, &F.pos_save, &F.r, &F.z, &F.p,
+    for (DevBuf* b : {&F.dinv_mk, &F.dinv_m, &F.bv, &F.vt, &F.dv, &F.v_it, &F.v_itp, &F.pos_save, &F.r, &F.z,
                       &F.q})
         b->reserve(sizeof(double) * vN);
     for (DevBuf* b : {&F.dinv_l, &F.bp, &F.pn, &F.p_itp}) b->reserve(sizeof(double) * (size_t)N);
     F.res_part.reserve(sizeof(double) * 4 * (size_t)pfem::frac_blocks(N));
-    F.part.reserve(sizeof(double) * 5 * (size_t)pfem::frac_blocks(D * N));
+    F.part.reserve(sizeof(double) * (4 * (size_t)pfem::frac_blocks(D * N) + pfem::kCgBlocks));
+    F.p.reserve(sizeof(double) * 2 * (size_t)D * (size_t)N);
     F.scal.reserve(sizeof(double) * 2);
     const size_t nq = sizeof(double) * (size_t)(D + 1) * N;
     c->q_prev.reserve(nq);
@@ -219,6 +222,7 @@ pfem::CgView frac_cg(pfem_case* c, int op, const double* vals, const double* b, 
     C.N = c->N;
     C.n = op == 0 ? c->N : c->dim * c->N;
     C.nb = pfem::frac_blocks(C.n);
+    C.nq = pfem::cg_blocks(C.N, C.dim);
     C.nbr_ptr = c->pat.nbr_ptr.as<int>();
     C.nbr_idx = c->pat.nbr_idx.as<int>();
     C.vals = vals;
@@ -248,7 +252,8 @@ int frac_cg_solve(pfem_case* c, const pfem::CgView& C, int* iters, double* relre
     int it = 0;
     while (std::isfinite(rr) && rr > thr && it < c->d.krylov_max_iter) {
         const int chunk = std::min(8, c->d.krylov_max_iter - it);
-        for (int k = 0; k < chunk; ++k, ++it) pfem::launch_cg2_iteration(C, it & 1, c->stream);
+        for (int k = 0; k < chunk; ++k, ++it) pfem::launch_cg2_iteration(C, it, c->stream);
+        pfem::launch_cg2_publish(C, c->stream);
         PFEM_HIP(hipMemcpyAsync(sc, C.scal, sizeof sc, hipMemcpyDeviceToHost, c->stream));
         PFEM_HIP(hipStreamSynchronize(c->stream));
         rr = sc[0];
@@ -1700,7 +1705,8 @@ int pfem_heat_step(pfem_case* c, double dt, pfem_step_stats* stats) {
         // iterations past convergence; CG keeps reducing the residual meanwhile)
         while (bb > 0 && std::isfinite(rr) && rr > thr && it < c->d.krylov_max_iter) {
             const int chunk = std::min(8, c->d.krylov_max_iter - it);
-            for (int k = 0; k < chunk; ++k, ++it) pfem::launch_cg_iteration(V, it & 1, c->stream);
+            for (int k = 0; k < chunk; ++k, ++it) pfem::launch_cg_iteration(V, it, c->stream);
+            pfem::launch_cg_publish(V, c->stream);
             PFEM_HIP(hipMemcpyAsync(sc, V.scal, sizeof sc, hipMemcpyDeviceToHost, c->stream));
             PFEM_HIP(hipStreamSynchronize(c->stream));
             rr = sc[0];

@@ -57,9 +57,10 @@ struct CgView {
     double* x = nullptr;
     double* r = nullptr;
     double* z = nullptr;
-    double* p = nullptr;
+    double* p = nullptr;     // [2][n] directions of the current and the previous iteration
     double* q = nullptr;
-    double* part = nullptr;  // [5][nb]: r.z (two parities), r.r, p.q, b.b
+    double* part = nullptr;  // [4][nb]: r.z (two parities), r.r, b.b; then [nq]: p.q
+    int nq = 0;              // workgroups of the product
     double* scal = nullptr;  // [2]: r.r, b.b after the last published pass
 };
 
@@ -73,6 +74,8 @@ void launch_frac_vstep(const FracView& V, hipStream_t s);
 // iterate = vt + dv, positions, residual partials; previous iterate <- iterate
 void launch_frac_update(const FracView& V, hipStream_t s);
 void launch_cg2_init(const CgView& C, hipStream_t s);
-void launch_cg2_iteration(const CgView& C, int par, hipStream_t s);
+// iteration it (from 0), with parity it & 1; launch_cg2_publish then gives the host r.r and b.b
+void launch_cg2_iteration(const CgView& C, int it, hipStream_t s);
+void launch_cg2_publish(const CgView& C, hipStream_t s);
 
 }  // namespace pfem

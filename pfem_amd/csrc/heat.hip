@@ -43,50 +43,58 @@ __global__ __launch_bounds__(kBlock) void k_heat_elem(HeatView V) {
     rec[15] = G.vol;
 }
 
-// one thread per node: its row of A = M + dt L (or the unit row) and, for a full row, its
-// share of b = sum_e M_e theta_prev (the diagonal entry's pair-element list holds every element
-// of the node, in element order)
-template <int D>
+// L lanes per node: its row of A = M + dt L (or the unit row) and, for a full row, its share of
+// b = sum_e M_e theta_prev.  The lanes take the row's off-diagonal entries (each the sum over its
+// pair-element list, in element order) and share the diagonal's list, which holds every element of
+// the node.  One thread per node walked ~100 element records in sequence (69k nodes, 3D: 249 ->
+// 83 us).
+template <int D, int L>
 __global__ __launch_bounds__(kBlock) void k_heat_asm(HeatView V) {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
+    const int i = (blockIdx.x * kBlock + threadIdx.x) / L, lane = threadIdx.x % L;
     if (i >= V.N) return;
     const uint8_t f = V.flags[i];
     const int rp = V.row_ptr[i];
     if ((f & V.dbit) || (f & NODE_FREE)) {
-        V.vals[rp] = 1.0;
+        if (lane == 0) V.vals[rp] = 1.0;
         return;
     }
     const double mfac = V.rho * V.cv / ((D + 1) * (D + 2));
     const int nb = V.nbr_ptr[i], deg = V.nbr_ptr[i + 1] - nb;
-    for (int k = 0; k < deg; ++k) {
+    auto term = [&](unsigned pe, double& vol, int& a) {  // an element's share of one entry
+        const int e = (int)(pe >> 4), bb = (int)(pe & 3u);
+        a = (int)((pe >> 2) & 3u);
+        const double* rec = V.erec + (size_t)kHeatRec * e;
+        vol = rec[15];
+        double gg = 0;
+#pragma unroll
+        for (int c = 0; c < D; ++c) gg += rec[c * (D + 1) + a] * rec[c * (D + 1) + bb];
+        return mfac * vol * (a == bb ? 2.0 : 1.0) + V.dt * (V.k * vol * gg);
+    };
+    double vol;
+    int a;
+    for (int k = lane; k < deg; k += L) {
         const int g = nb + k;
+        if (V.nbr_idx[g] == i) continue;
         double acc = 0.0;
-        for (int q = V.pei_ptr[g]; q < V.pei_ptr[g + 1]; ++q) {
-            const unsigned pe = V.pei[q];
-            const int e = (int)(pe >> 4), a = (int)((pe >> 2) & 3u), bb = (int)(pe & 3u);
-            const double* rec = V.erec + (size_t)kHeatRec * e;
-            const double vol = rec[15];
-            double gg = 0;
-#pragma unroll
-            for (int c = 0; c < D; ++c) gg += rec[c * (D + 1) + a] * rec[c * (D + 1) + bb];
-            acc += mfac * vol * (a == bb ? 2.0 : 1.0);
-            acc += V.dt * (V.k * vol * gg);
-        }
+        for (int q = V.pei_ptr[g]; q < V.pei_ptr[g + 1]; ++q) acc += term(V.pei[q], vol, a);
         V.vals[rp + k] = acc;
-        if (V.nbr_idx[g] == i) {
-            double bi = 0.0;
-            for (int q = V.pei_ptr[g]; q < V.pei_ptr[g + 1]; ++q) {
-                const unsigned pe = V.pei[q];
-                const int e = (int)(pe >> 4), a = (int)((pe >> 2) & 3u);
-                const double vol = V.erec[(size_t)kHeatRec * e + 15];
-                double t = 0;
+    }
+    const int kd = V.diag_pos[i] - rp, gd = nb + kd;
+    double acc = 0.0, bi = 0.0;
+    for (int q = V.pei_ptr[gd] + lane; q < V.pei_ptr[gd + 1]; q += L) {
+        const unsigned pe = V.pei[q];
+        acc += term(pe, vol, a);
+        double t = 0;
 #pragma unroll
-                for (int jj = 0; jj <= D; ++jj)
-                    t += mfac * vol * (jj == a ? 2.0 : 1.0) * V.Tprev[V.conn[(size_t)jj * V.E + e]];
-                bi += t;
-            }
-            V.b[i] = bi;
-        }
+        for (int jj = 0; jj <= D; ++jj)
+            t += mfac * vol * (jj == a ? 2.0 : 1.0) * V.Tprev[V.conn[(size_t)jj * V.E + (int)(pe >> 4)]];
+        bi += t;
+    }
+    acc = group_sum<L>(acc);
+    bi = group_sum<L>(bi);
+    if (lane == 0) {
+        V.vals[rp + kd] = acc;
+        V.b[i] = bi;
     }
 }
 
@@ -225,21 +233,33 @@ __global__ __launch_bounds__(kBlock) void k_heat_bc(HeatView V) {
 // Reductions are fence-free: every workgroup writes its partial sums to its own slot, and the
 // next kernel's workgroups re-reduce them in workgroup order.  rz partials alternate between
 // two arrays by iteration parity, so no kernel reads a slot that it also writes.
+// An iteration is two launches: Q finishes the previous one (beta, p = z + beta p_old) while it
+// multiplies, gathering z and p_old and adding A z + beta A p_old (the directions alternate between
+// two arrays, so no workgroup overwrites what another still gathers), X updates x, r and z.  Both
+// issue their loads before they sum the partials.  A group of lanes takes a row: one thread per row
+// read each value from another cache line.  69k nodes in 3D: three
+// launches 22 -> 14 us per iteration; what is left is the rows' values and two launches' latency.
 
-__device__ double sum_partials(const double* p, int nb) {
-    __shared__ double red[kBlock];
-    double s = 0;
-    for (int q = threadIdx.x; q < nb; q += kBlock) s += p[q];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = kBlock / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
+// Sums of two arrays of partials, in every thread.
+struct CgSums {
+    double v[2];
+    __device__ __forceinline__ void load(const double* a, int na, const double* b, int nb) {
+        v[0] = v[1] = 0.0;
+        for (int q = threadIdx.x; q < na; q += kBlock) v[0] += a[q];
+        for (int q = threadIdx.x; q < nb; q += kBlock) v[1] += b[q];
     }
-    const double r = red[0];
-    __syncthreads();
-    return r;
-}
+    __device__ __forceinline__ void sum() {
+        __shared__ double bc[2];
+        block_sum<2>(v);
+        if (threadIdx.x == 0) {
+            bc[0] = v[0];
+            bc[1] = v[1];
+        }
+        __syncthreads();
+        v[0] = bc[0];
+        v[1] = bc[1];
+    }
+};
 
 __device__ double row_dot(const HeatView& V, int i, const double* x) {
     double s = 0;
@@ -247,7 +267,7 @@ __device__ double row_dot(const HeatView& V, int i, const double* x) {
     return s;
 }
 
-// r = b - A x, z = D^-1 r, p = z; partials of r.z (parity 0), r.r and b.b
+// r = b - A x, z = D^-1 r; partials of r.z (parity 0), r.r and b.b
 __global__ __launch_bounds__(kBlock) void k_cg_init(HeatView V) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     double v[3] = {0, 0, 0};
@@ -256,7 +276,6 @@ __global__ __launch_bounds__(kBlock) void k_cg_init(HeatView V) {
         const double z = V.dinv[i] * r;
         V.r[i] = r;
         V.z[i] = z;
-        V.p[i] = z;
         v[0] = r * z;
         v[1] = r * r;
         v[2] = V.b[i] * V.b[i];
@@ -265,34 +284,61 @@ __global__ __launch_bounds__(kBlock) void k_cg_init(HeatView V) {
     if (threadIdx.x == 0) {
         V.part[blockIdx.x] = v[0];                    // rz, parity 0
         V.part[2 * V.nb + blockIdx.x] = v[1];         // rr
-        V.part[4 * V.nb + blockIdx.x] = v[2];         // bb
+        V.part[3 * V.nb + blockIdx.x] = v[2];         // bb
     }
 }
 
-// q = A p; partials of p.q
-__global__ __launch_bounds__(kBlock) void k_cg_q(HeatView V) {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    double v[1] = {0};
-    if (i < V.N) {
-        const double q = row_dot(V, i, V.p);
-        V.q[i] = q;
-        v[0] = V.p[i] * q;
+// Q: beta = rz_new / rz_old, p = z + beta p_old (first: p = z), q = A p; partials of p.q
+template <int L>
+__global__ __launch_bounds__(kBlock) void k_cg_q(HeatView V, int par, int first) {
+    constexpr int NPB = kBlock / L;
+    const double* __restrict__ z = V.z;
+    const double* __restrict__ po = first ? V.z : V.p + (size_t)(1 - par) * V.N;
+    double* pn = V.p + (size_t)par * V.N;
+    const int lane = threadIdx.x % L;
+    CgSums S;
+    S.load(V.part + par * V.nb, V.nb, V.part + (1 - par) * V.nb, V.nb);
+    double v[1] = {0}, beta = 0.0;
+    for (int i0 = blockIdx.x * NPB; i0 < V.N; i0 += gridDim.x * NPB) {
+        const int i = i0 + threadIdx.x / L, ic = min(i, V.N - 1);
+        double sz = 0, sp = 0;
+        for (int q = V.row_ptr[ic] + lane; q < V.row_ptr[ic + 1]; q += L) {
+            const int j = V.col[q];
+            const double a = V.vals[q];
+            sz += a * z[j];
+            sp += a * po[j];
+        }
+        sz = group_sum<L>(sz);
+        sp = group_sum<L>(sp);
+        const double zi = z[ic], pi = po[ic];
+        if (i0 == (int)blockIdx.x * NPB && !first) {
+            S.sum();
+            beta = S.v[1] != 0.0 ? S.v[0] / S.v[1] : 0.0;
+        }
+        if (i < V.N && lane == 0) {
+            const double p = zi + beta * pi, q = sz + beta * sp;
+            pn[i] = p;
+            V.q[i] = q;
+            v[0] += p * q;
+        }
     }
     block_sum<1>(v);
-    if (threadIdx.x == 0) V.part[3 * V.nb + blockIdx.x] = v[0];
+    if (threadIdx.x == 0) V.part[4 * V.nb + blockIdx.x] = v[0];
 }
 
-// alpha = rz / pq; x += alpha p; r -= alpha q; z = D^-1 r; partials of r.z (other parity), r.r
+// X: alpha = rz / pq; x += alpha p; r -= alpha q; z = D^-1 r; partials of r.z (other parity), r.r
 __global__ __launch_bounds__(kBlock) void k_cg_x(HeatView V, int par) {
-    const double rz = sum_partials(V.part + par * V.nb, V.nb);
-    const double pq = sum_partials(V.part + 3 * V.nb, V.nb);
-    const double alpha = pq != 0.0 ? rz / pq : 0.0;
-    const int i = blockIdx.x * kBlock + threadIdx.x;
+    const int i = blockIdx.x * kBlock + threadIdx.x, ic = min(i, V.N - 1);
+    CgSums S;
+    S.load(V.part + par * V.nb, V.nb, V.part + 4 * V.nb, V.nq);
+    const double x = V.x[ic], p = V.p[(size_t)par * V.N + ic], q = V.q[ic], r0 = V.r[ic], di = V.dinv[ic];
+    S.sum();
+    const double alpha = S.v[1] != 0.0 ? S.v[0] / S.v[1] : 0.0;
     double v[2] = {0, 0};
     if (i < V.N) {
-        V.x[i] += alpha * V.p[i];
-        const double r = V.r[i] - alpha * V.q[i];
-        const double z = V.dinv[i] * r;
+        V.x[i] = x + alpha * p;
+        const double r = r0 - alpha * q;
+        const double z = di * r;
         V.r[i] = r;
         V.z[i] = z;
         v[0] = r * z;
@@ -305,30 +351,14 @@ __global__ __launch_bounds__(kBlock) void k_cg_x(HeatView V, int par) {
     }
 }
 
-// beta = rz_new / rz_old; p = z + beta p; workgroup 0 publishes r.r and b.b for the host
-__global__ __launch_bounds__(kBlock) void k_cg_p(HeatView V, int par) {
-    const double rz_old = sum_partials(V.part + par * V.nb, V.nb);
-    const double rz_new = sum_partials(V.part + (1 - par) * V.nb, V.nb);
-    const double beta = rz_old != 0.0 ? rz_new / rz_old : 0.0;
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < V.N) V.p[i] = V.z[i] + beta * V.p[i];
-    if (blockIdx.x == 0) {
-        const double rr = sum_partials(V.part + 2 * V.nb, V.nb);
-        const double bb = sum_partials(V.part + 4 * V.nb, V.nb);
-        if (threadIdx.x == 0) {
-            V.scal[0] = rr;
-            V.scal[1] = bb;
-        }
-    }
-}
-
-// the initial r.r and b.b (before any iteration)
+// r.r and b.b for the host
 __global__ __launch_bounds__(kBlock) void k_cg_publish(HeatView V) {
-    const double rr = sum_partials(V.part + 2 * V.nb, V.nb);
-    const double bb = sum_partials(V.part + 4 * V.nb, V.nb);
+    CgSums S;
+    S.load(V.part + 2 * V.nb, V.nb, V.part + 3 * V.nb, V.nb);
+    S.sum();
     if (threadIdx.x == 0) {
-        V.scal[0] = rr;
-        V.scal[1] = bb;
+        V.scal[0] = S.v[0];
+        V.scal[1] = S.v[1];
     }
 }
 
@@ -340,11 +370,11 @@ void launch_heat_assemble(const HeatView& V, hipStream_t s) {
     const int be = heat_blocks(V.E), bn = heat_blocks(V.N), bf = heat_blocks(V.F);
     if (V.dim == 2) {
         k_heat_elem<2><<<be, kBlock, 0, s>>>(V);
-        k_heat_asm<2><<<bn, kBlock, 0, s>>>(V);
+        k_heat_asm<2, 8><<<heat_blocks(V.N * 8), kBlock, 0, s>>>(V);
         if (V.F > 0) k_heat_facet<2><<<bf, kBlock, 0, s>>>(V);
     } else {
         k_heat_elem<3><<<be, kBlock, 0, s>>>(V);
-        k_heat_asm<3><<<bn, kBlock, 0, s>>>(V);
+        k_heat_asm<3, 16><<<heat_blocks(V.N * 16), kBlock, 0, s>>>(V);
         if (V.F > 0) k_heat_facet<3><<<bf, kBlock, 0, s>>>(V);
     }
     k_heat_bc<<<bn, kBlock, 0, s>>>(V);
@@ -352,13 +382,15 @@ void launch_heat_assemble(const HeatView& V, hipStream_t s) {
 
 void launch_cg_init(const HeatView& V, hipStream_t s) {
     k_cg_init<<<V.nb, kBlock, 0, s>>>(V);
-    k_cg_publish<<<1, kBlock, 0, s>>>(V);
+    launch_cg_publish(V, s);
 }
 
-void launch_cg_iteration(const HeatView& V, int par, hipStream_t s) {
-    k_cg_q<<<V.nb, kBlock, 0, s>>>(V);
-    k_cg_x<<<V.nb, kBlock, 0, s>>>(V, par);
-    k_cg_p<<<V.nb, kBlock, 0, s>>>(V, par);
+void launch_cg_iteration(const HeatView& V, int it, hipStream_t s) {
+    if (V.dim == 2) k_cg_q<kCgLanes[0]><<<V.nq, kBlock, 0, s>>>(V, it & 1, it == 0);
+    else k_cg_q<kCgLanes[1]><<<V.nq, kBlock, 0, s>>>(V, it & 1, it == 0);
+    k_cg_x<<<V.nb, kBlock, 0, s>>>(V, it & 1);
 }
+
+void launch_cg_publish(const HeatView& V, hipStream_t s) { k_cg_publish<<<1, kBlock, 0, s>>>(V); }
 
 }  // namespace pfem

@@ -37,16 +37,28 @@ struct HeatView {
     double* x = nullptr;
     double* r = nullptr;
     double* z = nullptr;
-    double* p = nullptr;
+    double* p = nullptr;     // [2][N] directions of the current and the previous iteration
     double* q = nullptr;
     double* dinv = nullptr;
-    double* part = nullptr;  // [5][nb]: r.z (two parities), r.r, p.q, b.b
+    double* part = nullptr;  // [4][nb]: r.z (two parities), r.r, b.b; then [nq]: p.q
+    int nq = 0;              // workgroups of the product
     double* scal = nullptr;  // [2]: r.r, b.b after the last published pass
 };
+
+// Lanes per node of the conjugate gradients' products (a node's ~7 / ~15 neighbours in 2D / 3D) and
+// their workgroups (grid-stride, so that the next kernel's workgroups sum few partials).
+constexpr int kCgLanes[2] = {4, 8};
+constexpr int kCgBlocks = 1024;
+inline int cg_blocks(int n, int dim) {
+    const int per = 256 / kCgLanes[dim - 2];
+    return n < per * kCgBlocks ? (n + per - 1) / per : kCgBlocks;
+}
 
 int heat_blocks(int n);
 void launch_heat_assemble(const HeatView& V, hipStream_t s);
 void launch_cg_init(const HeatView& V, hipStream_t s);
-void launch_cg_iteration(const HeatView& V, int par, hipStream_t s);
+// iteration it (from 0), with parity it & 1; launch_cg_publish then gives the host r.r and b.b
+void launch_cg_iteration(const HeatView& V, int it, hipStream_t s);
+void launch_cg_publish(const HeatView& V, hipStream_t s);
 
 }  // namespace pfem
