@@ -386,6 +386,7 @@ struct Engine::Impl {
     SlotScal* h_reset = nullptr;  // staging of host-written slot scalars
     BlockTask* h_tab = nullptr;
     size_t tab_cap = 0;
+    size_t tab_sent = 0;  // leading entries of h_tab that the device holds
     std::vector<int> free_slots;
     int par = 0;
     bool prof = false;
@@ -1126,7 +1127,7 @@ void Engine::tick(std::vector<Req*>& done) {
         // the step's own kernels give the CFL minimum after it; the CFL pass runs on its own
         // only without a step
         if ((op & OP_CFL) && !(op & OP_WC)) append(tab[(c->dim == 2 ? T_CFE2 : T_CFE3) + wi], sl, c->E, kElemCap);
-        if (op & (OP_WC | OP_CFL)) {
+        if ((op & OP_CFL) && !(op & OP_WC)) {  // (a step's first kernel sets it)
             SlotScal& h = I.h_reset[sl];
             h.dt2 = 0x7fefffffffffffffULL;  // DBL_MAX
             PFEM_HIP(hipMemcpyAsync(&I.dslot(sl)->dt2, &h.dt2, sizeof(h.dt2), hipMemcpyHostToDevice, s));
@@ -1140,10 +1141,22 @@ void Engine::tick(std::vector<Req*>& done) {
         I.tab_cap = std::max<size_t>(total * 2, 4096);
         pinned_alloc(I.h_tab, I.tab_cap);
         I.d_tab.reserve(sizeof(BlockTask) * I.tab_cap);
+        I.tab_sent = 0;
     }
-    for (int t = 0; t < T_NTAB; ++t)
-        if (!tab[t].empty()) std::memcpy(I.h_tab + off[t], tab[t].data(), sizeof(BlockTask) * tab[t].size());
-    if (total) PFEM_HIP(hipMemcpyAsync(I.d_tab.p, I.h_tab, sizeof(BlockTask) * total, hipMemcpyHostToDevice, s));
+    // sent only where the device does not hold the same tables from the tick before (an explicit
+    // step repeats them every time); h_tab is what it holds
+    bool same = total <= I.tab_sent;
+    for (int t = 0; t < T_NTAB; ++t) {
+        const size_t bytes = sizeof(BlockTask) * tab[t].size();
+        if (!bytes || (same && std::memcmp(I.h_tab + off[t], tab[t].data(), bytes) == 0)) continue;
+        same = false;
+        std::memcpy(I.h_tab + off[t], tab[t].data(), bytes);
+    }
+    if (!same) {
+        I.tab_sent = 0;
+        PFEM_HIP(hipMemcpyAsync(I.d_tab.p, I.h_tab, sizeof(BlockTask) * total, hipMemcpyHostToDevice, s));
+        I.tab_sent = total;
+    }
     auto T = [&](int t) { return I.d_tab.as<BlockTask>() + off[t]; };
     auto NT = [&](int t) { return (int)tab[t].size(); };
 
