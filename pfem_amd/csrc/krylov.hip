@@ -24,9 +24,9 @@
 //          (t, t), (rh, t)
 // U also sums (r, r), which the test after V reads.  (Five launches per iteration before, with
 // field-blocked vectors; each is a chain of dependent loads that takes ~5 us on a small system.
-// Per iteration: 1,001 nodes in 2D 29 -> 16 us, 12k nodes in 3D 59 -> 31 us, 48k Delaunay nodes
-// 94 -> 76 us, 72k nodes with FP32 inner solves 68 -> 49 us; above 100k nodes the products are
-// bound by the matrix's bytes.)
+// Per iteration: 1,001 nodes in 2D 29 -> 15 us, 12k nodes in 3D 59 -> 25 us, 48k Delaunay nodes
+// 94 -> 61 us, 72k nodes with FP32 inner solves 68 -> 43 us, the last three with plain value loads
+// (ELL_STREAM); above 100k nodes the products are bound by the matrix's bytes.)
 //
 // Reductions: every workgroup writes its FP64 partial sums to its own place and the next
 // kernel's workgroups each re-reduce them in block order — deterministic, and ordered by
