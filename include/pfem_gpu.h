@@ -138,7 +138,7 @@ typedef struct pfem_solve_stats {
     int32_t status;       /* PFEM_OK / PFEM_NOT_CONVERGED / PFEM_NAN */
     int32_t krylov_iters; /* BiCGSTAB iterations (inner iterations in mixed mode) */
     int32_t refinements;  /* FP64 refinement sweeps (mixed mode) */
-    int32_t restarts;
+    int32_t restarts;     /* BiCGSTAB restarts after a breakdown or a rho lost in rounding, and fallbacks to FP64 */
     double relres;        /* final ||b - A x|| / ||b|| in FP64 */
 } pfem_solve_stats;
 

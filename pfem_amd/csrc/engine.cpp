@@ -718,6 +718,7 @@ void Engine::Impl::reset_kscal(int slot, int which, double rtol, int maxit, doub
 void Engine::Impl::restart_kscal(int slot, int which) {
     KScal& k = h_reset[slot].k[which];
     k = h_scal[slot].k[which];
+    if (k.done == 4) k.weak++;
     k.done = 0;
     k.req_init = 1;
     PFEM_HIP(hipMemcpyAsync(&dslot(slot)->k[which], &k, sizeof(KScal), hipMemcpyHostToDevice, s));
@@ -1372,8 +1373,8 @@ void Engine::tick(std::vector<Req*>& done) {
                         r->verifying = true;
                         I.restart_kscal(r->slot, 0);
                         r->ops = OP_K64_INIT | OP_K64_RUN;
-                    } else if (k.done == 2 && r->restarts < 8 && k.iters < k.maxit) {
-                        r->restarts++;
+                    } else if (k.done == 4 || (k.done == 2 && r->restarts < 8 && k.iters < k.maxit)) {
+                        if (k.done == 2) r->restarts++;
                         I.restart_kscal(r->slot, 0);
                         r->ops = OP_K64_INIT | OP_K64_RUN;
                     } else {
@@ -1381,7 +1382,7 @@ void Engine::tick(std::vector<Req*>& done) {
                         if (k.done == 2) stt = PFEM_NAN;
                         else if (k.done == 3) stt = (k.bb > 0 && std::isfinite(k.rr)) ? PFEM_NOT_CONVERGED : PFEM_NAN;
                         r->ss.krylov_iters += k.iters;
-                        r->ss.restarts += r->restarts + (r->fallback ? 1 : 0);
+                        r->ss.restarts += r->restarts + k.weak + (r->fallback ? 1 : 0);
                         r->ss.relres = k.bb > 0 ? std::sqrt(k.rr / k.bb) : 0.0;
                         solve_done(I, r, stt);
                     }

@@ -9,9 +9,9 @@
 // The vector updates are merged into as few launches as the two reductions of an iteration
 // allow.  rho is taken from the previous product as (rh, s) - omega (rh, t) (as in the improved
 // BiCGSTAB of Yang and Brent 2002), so that the end of one iteration and the start of the next
-// are one pass; and with block Jacobi the preconditioned vectors follow the recurrences of the
-// plain ones (rhat = B^-1 r and vhat = B^-1 v are local to a node), so that the products read
-// them from there.  One iteration is
+// are one pass (a rho lost in rounding ends it: kWeakRho in views.hpp); and with block Jacobi the
+// preconditioned vectors follow the recurrences of the plain ones (rhat = B^-1 r and vhat = B^-1 v
+// are local to a node), so that the products read them from there.  One iteration is
 //   block Jacobi (3 launches)                   multigrid M (4 launches and two V-cycles)
 //   U: r = s - om t, s = r - al v;              U: the same, with s stored;
 //      x += al ph + om (rhat - al vhat);           x += al ph + om sh;
@@ -150,6 +150,8 @@ __global__ __launch_bounds__(kBlock) void k_kry_init_fin(const KrylovView<T>* __
             S.tol2 = S.rtol * S.rtol * tot[2];
             if (S.atol2 > 0.0 && S.atol2 < S.tol2) S.tol2 = S.atol2;
             S.rr = tot[1];
+            // (rh = r here)
+            S.weak_rho = sizeof(T) == 8 && S.weak < kMaxWeak ? kWeakRho * sqrt(tot[1]) : -1.0;
             S.slot[par].rho = tot[0];
             S.slot[par].alpha = 1.0;
             S.slot[par].omega = 1.0;
@@ -354,13 +356,16 @@ __device__ __forceinline__ bool step_alpha(const KrylovView<T>& V, const BlockTa
     KScal& S = *V.sc;
     constexpr int rs[2] = {P_RV, P_RR};
     double tot[2];
+    // (loaded ahead of the reduction: loads in the tests below are waited for one by one)
+    const double rho = S.slot[par].rho, tol2 = S.tol2, weak_rho = S.weak_rho;
+    const int state = S.slot[par].state, iters = S.iters, maxit = S.maxit;
     reduce_partials<2>(V.partials, V.nblk, rs, tot);
-    const int state = S.slot[par].state;
-    alpha = S.slot[par].rho / tot[0];
+    alpha = rho / tot[0];
     int stop = 0;
-    if (state == K_CONV || tot[1] <= S.tol2) stop = 1;
+    if (state == K_CONV || tot[1] <= tol2) stop = 1;
     else if (state == K_BREAK || !isfinite(tot[1])) stop = 2;
-    else if (S.iters >= S.maxit) stop = 3;
+    else if (iters >= maxit) stop = 3;
+    else if (fabs(rho) <= weak_rho * sqrt(tot[1])) stop = 4;
     else if (tot[0] == 0.0 || !isfinite(alpha)) stop = 2;
     if (task.block == 0 && threadIdx.x == 0) {
         S.rr = tot[1];

@@ -133,16 +133,31 @@ struct KScal {
     KSlot slot[2];
     double rr;    // last ||r||^2
     double bb;    // ||b||^2
+    double weak_rho;  // rho is lost at |rho| <= weak_rho ||r|| (set by init; negative: not tested)
     double tol2;  // absolute squared tolerance on ||r||^2
     double rtol;
     double atol2; // > 0: ||r||^2 must also fall below it (absolute cap), 0: relative only
-    int done;     // 0 running, 1 converged, 2 breakdown or non-finite, 3 iteration limit
+    int done;     // 0 running, 1 converged, 2 breakdown or non-finite, 3 iteration limit, 4 rho lost
+                  // in rounding (kWeakRho): the host restarts with a new shadow residual
     int iters;
     int maxit;
     int req_init;  // set by the host: the next init launch (re)starts this case
     int true_rr;   // 1 when rr is a true residual b - A x (set by init, cleared by each iteration)
-    int pad;
+    int weak;      // restarts on a lost rho so far (after kMaxWeak the solve goes on without the test)
 };
+
+// An FP64 solve's rho = (rh, r) is taken for lost at |rho| <= kWeakRho ||rh|| ||r||, the unit
+// roundoff: beta and alpha are then rounding noise, and the solve wanders on a plateau for
+// thousands of iterations (what ends it otherwise, rho = 0 exactly, only a dot product meets, whose
+// rounding lies on a grid; the recurrence for rho never does).  Iterations per case without the
+// test / at 1e-17 / 1e-16 / 1e-15, block Jacobi to a relative residual of 1e-10: 3D column fields of
+// 72k nodes (two steps) 1,240 / 1,152 / 1,081 / 1,022, 250k (one) 1,549 / 1,062 / 1,011 / 882, 1.03M (one)
+// 3,915 / - / 1,654 / 1,487; 8k nodes in 2D 1,981 / 1,973 / 1,873 / 1,680; a dam break of 1k nodes to
+// 1e-12 838 / 838 / 838 / 849 (0.05, 0.25 and 0.5 restarts per step; one idles the rest of its launches:
+// 18.5, 18.7 and 19.1 ms).  FP32 inner solves end at their own limits: with the test at 1e-11, their
+// rounding, 72k nodes took 1,450 iterations instead of 1,366.
+constexpr double kWeakRho = 1.1102230246251565e-16;
+constexpr int kMaxWeak = 64;
 
 // The per-workgroup partial sums: kPartStride arrays of kMaxCaseBlocks doubles per case.
 enum : int { P_RR = 0, P_RV = 1, P_SS = 2, P_TS = 3, P_TT = 4, P_RHT = 5, P_RHS = 6, P_RHR = 2, P_BB = 3, kPartStride = 8 };
