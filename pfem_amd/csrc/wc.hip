@@ -43,6 +43,8 @@ constexpr double kRefSize = D == 2 ? 0.5 : 0.16666666666666666666666666666667;  
 // node's shape function (3D: the cross products of the edges, area vectors of the faces through
 // the node; C, their sum, is minus the own node's, the area vector of the opposite face), so a
 // visit needs one division in all (1 / det J) and no gradient selection by local index.
+// The products' roundings are spelled out (fma): he of one element in one node's frame must have the
+// same bits in the step and in the CFL pass, whatever the compiler merges around it.
 template <int D>
 struct Frame {
     double c[D][D], C[D], dj;
@@ -57,9 +59,9 @@ __device__ __forceinline__ void frame_of(const double (&e)[D][D], Frame<D>& F) {
         F.c[1][1] = e[0][0];
     } else {
         auto cross = [](const double (&u)[D], const double (&v)[D], double (&w)[D]) {
-            w[0] = u[1] * v[D - 1] - u[D - 1] * v[1];
-            w[1] = u[D - 1] * v[0] - u[0] * v[D - 1];
-            w[D - 1] = u[0] * v[1] - u[1] * v[0];
+            w[0] = fma(u[1], v[D - 1], -(u[D - 1] * v[1]));
+            w[1] = fma(u[D - 1], v[0], -(u[0] * v[D - 1]));
+            w[D - 1] = fma(u[0], v[1], -(u[1] * v[0]));
         };
         cross(e[1], e[D - 1], F.c[0]);
         cross(e[D - 1], e[0], F.c[1]);
@@ -68,7 +70,7 @@ __device__ __forceinline__ void frame_of(const double (&e)[D][D], Frame<D>& F) {
     F.dj = 0;
 #pragma unroll
     for (int k = 0; k < D; ++k) {
-        F.dj += e[0][k] * F.c[0][k];
+        F.dj = fma(e[0][k], F.c[0][k], F.dj);
         F.C[k] = F.c[0][k];
 #pragma unroll
         for (int m = 1; m < D; ++m) F.C[k] += F.c[m][k];
@@ -78,8 +80,8 @@ __device__ __forceinline__ void frame_of(const double (&e)[D][D], Frame<D>& F) {
 // he = 2 r_in of an element (Element::getRin, Element.cpp:226-294): 2D |e| / semi-perimeter,
 // 3D 3 |e| / total face area; the edges' (2D) or faces' (3D) measures are the frame's lengths.
 //
-// The square roots take the hardware's reciprocal square root estimate through Goldschmidt's
-// iteration (two steps and a residual correction: within an ulp); the library's adds range
+// The square roots take the hardware's reciprocal square root estimate through one coupled step of
+// Goldschmidt's iteration and two residual corrections (within an ulp); the library's adds range
 // scaling that areas and lengths of elements do not need.  2^-1000 keeps a zero finite.
 __device__ __forceinline__ double sqrt_len(double v) {
     v = fmax(v, 9.332636185032189e-302);
@@ -101,7 +103,7 @@ __device__ __forceinline__ double elem_he(const Frame<D>& F) {
 #pragma unroll
         for (int k = 0; k < D; ++k) {
             const double v = m < D ? F.c[m < D ? m : 0][k] : F.C[k];
-            q += v * v;
+            q = fma(v, v, q);
         }
         s += sqrt_len(q);
     }
@@ -111,13 +113,15 @@ __device__ __forceinline__ double elem_he(const Frame<D>& F) {
 // One node's share of computeNextDT (WCompNewton/Solver.cpp:192-234) through an element of
 // size he: sc^2 he^2 / max(u^2, c^2, 4 alpha^2 / he^2) with c^2 = (K0 + K0' p) / rho
 // (ContEquation.inl:117-121), alpha = mu / rho (MomEquation.inl:184-198).  The reference's
-// element value is the smallest of its nodes' shares (x / max(a, b) = min(x / a, x / b) in
-// correctly rounded arithmetic), and a share only grows with he, so a node's smallest share
-// over its elements is the one through its smallest he: the minimum over nodes of that
-// equals the reference's minimum over elements, bit for bit.
+// element value is the smallest of its nodes' shares (x / max(a, b) = min(x / a, x / b)), and a
+// share only grows with he, so a node's smallest share over its elements is the one through its
+// smallest he.  The step takes the minimum over nodes of that and the CFL pass the minimum over
+// every element's nodes; both evaluate he in the frame of the share's node (an element's frames
+// round it differently) and agree bit for bit, so that a run restarted from saved states and
+// positions takes the time steps of an uninterrupted one.
 __device__ __forceinline__ double cfl_share(double sc2, double he, double u2, double p, double rho, double K0,
                                             double K0p, double mu) {
-    const double c2 = (K0 + K0p * p) / rho;
+    const double c2 = fma(K0p, p, K0) / rho;
     const double alpha = mu / rho;
     const double maxS = fmax(fmax(u2, c2), 4 * alpha * alpha / (he * he));
     return sc2 * he * he / maxS;
@@ -386,7 +390,7 @@ __device__ __forceinline__ double wc_finish(const WcView<S>& V, int i, uint8_t f
         V.a[q] = (S)acc;
         const S vs = (S)((double)V.vh[q] + 0.5 * V.dt * acc);
         V.v[q] = vs;
-        u2 += (double)vs * (double)vs;
+        u2 = fma((double)vs, (double)vs, u2);
     }
     if (f & NODE_FREE) return 1.7976931348623157e308;
     return cfl_share(V.sc2, hmin, u2, (double)V.p[i], (double)V.rho[i], V.K0, V.K0p, V.mu);
@@ -526,7 +530,8 @@ __global__ __launch_bounds__(kBlock) void k_wc_mom_node(const WcView<S>* __restr
 }
 
 // CFL on its own (no step before it): dt^2 = min_e sc^2 he^2 / max_n(u^2, c^2, 4 alpha^2/he^2),
-// he = 2 r_in (Element.cpp:226-294), as the minimum of every element node's share.
+// he = 2 r_in (Element.cpp:226-294), as the minimum of every element node's share, through he in
+// that node's frame.
 template <int D, typename S>
 __global__ __launch_bounds__(kBlock) void k_wc_cfl(const WcView<S>* __restrict__ views,
                                                    const BlockTask* __restrict__ tasks) {
@@ -541,25 +546,28 @@ __global__ __launch_bounds__(kBlock) void k_wc_cfl(const WcView<S>* __restrict__
         int nd[NE];
 #pragma unroll
         for (int a = 0; a < NE; ++a) nd[a] = V.conn[(long long)a * E + e];
-        double ed[D][D];
+        double x[NE][D];
 #pragma unroll
-        for (int a = 1; a < NE; ++a)
+        for (int a = 0; a < NE; ++a)
 #pragma unroll
-            for (int k = 0; k < D; ++k)
-                ed[a - 1][k] = V.pos[(long long)k * N + nd[a]] - V.pos[(long long)k * N + nd[0]];
-        Frame<D> F;
-        frame_of<D>(ed, F);
-        const double he = elem_he<D>(F);
+            for (int k = 0; k < D; ++k) x[a][k] = V.pos[(long long)k * N + nd[a]];
 #pragma unroll
         for (int a = 0; a < NE; ++a) {
+            double ed[D][D];
+#pragma unroll
+            for (int m = 1; m < NE; ++m)
+#pragma unroll
+                for (int k = 0; k < D; ++k) ed[m - 1][k] = x[wc_other<D>(a, m)][k] - x[a][k];
+            Frame<D> F;
+            frame_of<D>(ed, F);
             const int i = nd[a];
             double u2 = 0;
 #pragma unroll
             for (int k = 0; k < D; ++k) {
                 const double vk = (double)V.v[(long long)k * N + i];
-                u2 += vk * vk;
+                u2 = fma(vk, vk, u2);
             }
-            best = fmin(best, cfl_share(sc2, he, u2, (double)V.p[i], (double)V.rho[i], V.K0, V.K0p, V.mu));
+            best = fmin(best, cfl_share(sc2, elem_he<D>(F), u2, (double)V.p[i], (double)V.rho[i], V.K0, V.K0p, V.mu));
         }
     }
     block_min_to(V.dt2, best);
