@@ -1270,9 +1270,7 @@ int pfem_bench_kernels(pfem_case* c, int32_t reps, double* out10) {
             kv.v = w + n;
             kv.s = w + 2LL * n;
             kv.partials = c->partials.as<double>();
-            pfem::KScal sc{};  // a running solve: (r, r) = 0 is above this tolerance
-            sc.tol2 = -1.0;
-            sc.maxit = 1;
+            const pfem::KScal sc{};  // done = 0: the kernel runs
             DevBuf d_tasks, d_view, d_sc;
             d_tasks.reserve(sizeof(pfem::BlockTask) * tasks.size());
             d_view.reserve(sizeof(kv));
@@ -1303,8 +1301,8 @@ int pfem_bench_kernels(pfem_case* c, int32_t reps, double* out10) {
         out8[5] = (double)nnz;
         out8[6] = (double)c->pat.graph_nnz;
         out8[7] = (double)c->lanes;
-        if (c->amg.levels > 1) {  // the multigrid's level-0 residual t = r - A w over the FP64 ELL copy
-            const int nb = (int)std::min<long long>((c->N + pfem::kBlock - 1) / pfem::kBlock, 8192);
+        if (c->amg.levels > 1) {  // the multigrid's level-0 residual t = r - A w of an FP64 hierarchy
+            const int nb = pfem::kry_blocks(c->pat.ell_nsl);
             std::vector<pfem::BlockTask> tasks((size_t)nb);
             for (int b = 0; b < nb; ++b) tasks[(size_t)b] = pfem::BlockTask{0, b, nb, 0};
             DevBuf d_tasks, d_view, d_done;
@@ -1319,6 +1317,9 @@ int pfem_bench_kernels(pfem_case* c, int32_t reps, double* out10) {
             av.E0.soff = c->pat.ell_soff.as<int>();
             av.E0.idx = c->pat.ell_idx.as<int>();
             av.E0.vals = c->ws.vals_ell;
+            if (pfem::amg_l0_fp32(c))
+                av.E0f = {av.E0.N, av.E0.nf, av.E0.nsl, av.E0.ncol, av.E0.soff, av.E0.idx, c->ws.vals32_ell};
+            av.split = pfem::split_slices(c->pat.ell_nsl);
             av.level = 0;
             av.lanes = c->lanes;
             av.mask = 1;

@@ -188,6 +188,8 @@ bool amg_fp32(const pfem_case* c) {
     return c->amg_all_fp32 && c->d.precision == PFEM_PREC_MIXED && c->amg.levels > 1 && c->dim == 3;
 }
 
+}  // namespace
+
 // PFEM_PREC_MIXED cases otherwise keep the FP64 hierarchy but read FP32 values at level 0:
 // the residual t = r - A w (an FP32 ELL copy of the system) and the post-smoothing product
 // (A P) z (A P held in FP32), with FP64 vectors and sums.  The iteration counts do not
@@ -196,6 +198,8 @@ bool amg_fp32(const pfem_case* c) {
 bool amg_l0_fp32(const pfem_case* c) {
     return c->d.precision == PFEM_PREC_MIXED && c->amg.levels > 1 && !amg_fp32(c);
 }
+
+namespace {
 
 WsLayout ws_layout(const pfem_case* c) {
     WsLayout L{};

@@ -205,6 +205,7 @@ int row_blocks(long long n, int nsl = 0);
 bool split_slices(int nsl);
 int kry_blocks(int nsl);
 bool stream_values(long long value_bytes);
+bool amg_l0_fp32(const pfem_case* c);  // an FP64 hierarchy that reads FP32 values at level 0
 int pick_lanes(double avg_deg);
 
 }  // namespace pfem
