@@ -58,8 +58,9 @@ enum Tab : int {
 };
 
 // Multigrid tables of one hierarchy type, relative to T_AMG + type * A_N: setup per level
-// (Galerkin, block Jacobi), coarsest dense inverse; V-cycle per level (node ops, SpMV ops,
-// restriction), coarsest solve.
+// (Galerkin, block Jacobi, A P), coarsest dense inverse; V-cycle per level (slices of the level-0
+// residual and of every level's post-smoothing, aggregates of the coarser levels' residual with
+// restriction, level 0's restriction), coarsest solve with the level above it.
 enum AmgTab : int {
     A_G = 0, A_B = A_G + kAmgMaxLevels, A_D = A_B + kAmgMaxLevels, A_AP = A_D + 1,
     A_VN = A_AP + kAmgMaxLevels, A_VS = A_VN + kAmgMaxLevels, A_VR = A_VS + kAmgMaxLevels,
@@ -141,8 +142,9 @@ int row_blocks(long long n, int nsl) {
 // (72k, 3D FP32) 67 / 54, 4,110 (263k, 3D FP64) 260 / 228.
 bool split_slices(int nsl) { return nsl <= 768; }
 
-// While a launch's matrices leave half of the 256 MB memory-side cache free they are read with
-// plain loads: the non-temporal ones pass it by.  Product with plain / non-temporal loads: 12k nodes
+// While a launch's system matrices take at most 160 of the 256 MB memory-side cache (the
+// multigrid's copies, which the same flag governs, are not counted: the limit is empirical) they are
+// read with plain loads: the non-temporal ones pass it by.  Product with plain / non-temporal loads: 12k nodes
 // (3D FP64, 24 MB) 9.4 / 12.2 us, 72k FP32 (69 MB) 15.2 / 18.8, 60k FP64 (115 MB) 19.9 / 22.6; at
 // 110k (211 MB) 40.7 / 40.6, with the multigrid's other kernels 15 % slower for want of the cache.
 bool stream_values(long long value_bytes) { return value_bytes > (160LL << 20); }
@@ -175,11 +177,6 @@ struct WsLayout {
     size_t amg_lv[kAmgMaxLevels][6];
     size_t amg_ap[kAmgMaxLevels];  // A P values of level l (rows) against level l+1
 };
-// The multigrid hierarchy runs in FP32 for PFEM_PREC_MIXED 3D cases (under FP64 BiCGSTAB):
-// the 3D iteration counts did not change, and the all-FP32 3D hierarchy served the stream
-// 8 % faster than FP32 operators with FP64 vectors.  2D hierarchies keep FP64 vectors: an
-// FP32 V-cycle raised the 2D BiCGSTAB iteration count by 20-40 % (their level 0 reads FP32
-// values instead, amg_l0_fp32).
 // A hierarchy wholly in FP32 (values, inverses and vectors of every level): only for 3D
 // PFEM_PREC_MIXED cases set up with PFEM_AMG_FP32=1.  On the 512-request serving stream it
 // takes more BiCGSTAB iterations than an FP64 hierarchy with FP32 level-0 values (below):

@@ -19,9 +19,10 @@
 // applied to each velocity component: the reference's M is block diagonal with equal blocks,
 // and its unit rows and columns are per node).  One gather pass per node writes all three rows
 // and the prediction right-hand side from one element record per element, summing the
-// contributions of the elements holding both nodes in element order (the reference's triplet
-// order); the boundary conditions are applied in the same pass, row by row, in the reference's
-// order (Dirichlet columns by increasing node, then component).
+// contributions of the elements holding both nodes: off-diagonal values in element order, diagonal
+// values and right-hand sides in a fixed order, split over the node's lanes.  The boundary
+// conditions are applied in the same pass (each lane eliminates the Dirichlet columns among its
+// entries, the node's sum joins the lanes').
 #include "common.hpp"
 #include "fracstep.hpp"
 #include "heat.hpp"

@@ -12,9 +12,10 @@
 // Layout: a scalar CSR over the case's node graph (a full row holds the sorted neighbours,
 // the node itself included, so value k of row i is node-graph entry k of i; other rows hold
 // their diagonal only).  The assembly gathers, like the PSPG one: each value sums the
-// contributions of the elements holding both nodes (pair-element incidence, element order:
-// M_e then dt L_e per element, the order of the reference's triplet list), from one element
-// record per element (gradients and measure) written by an element pass.
+// contributions M_e + dt L_e of the elements holding both nodes (pair-element incidence) from one
+// element record per element (gradients and measure) written by an element pass: off-diagonal
+// values in element order, diagonal values and the right-hand side in a fixed order, split over
+// the node's lanes.
 #include "common.hpp"
 #include "heat.hpp"
 #include "p1geom.hpp"

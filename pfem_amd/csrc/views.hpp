@@ -13,8 +13,7 @@ namespace pfem {
 // vector registers, and is waited for together with every other access in flight.  Held as a
 // pointer into global memory, accesses through it are global ones.  Measured
 // (same bits): steps of a 12k-node 3D column 16.65 -> 16.24 ms, of a 48k-node Delaunay mesh 66.4 ->
-// 64.1 ms, of a 20k-node 2D column 27.95 -> 27.37 ms; the compressible tile passes, which also
-// use the LDS, 537 -> 443 us.
+// 64.1 ms, of a 20k-node 2D column 27.95 -> 27.37 ms.
 #if defined(__HIP_DEVICE_COMPILE__)
 #define PFEM_GLOBAL __attribute__((address_space(1)))
 #else
@@ -280,7 +279,7 @@ struct RefineView {
 
 // Tiles of the weakly compressible passes (2D, 3D): consecutive nodes per workgroup, lanes per
 // node (a P1 node has ~6 incident triangles in 2D and ~24 tetrahedra in 3D), the nodes that one
-// tile stages in LDS at most (72 bytes each in FP64) and the visit words staged beside them:
+// tile stages in LDS at most (64 bytes each in FP64, 3D momentum pass) and the visit words staged beside them:
 // together with the static arrays within 64 KiB.  Tiles of a spatially ordered 3D mesh hold ~600
 // nodes, of a random order up to ~1,000; elements with a node beyond the capacity are visited
 // through memory (kWcFar), visit words past theirs are read from memory.

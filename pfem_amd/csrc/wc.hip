@@ -10,8 +10,9 @@
 //
 // Tile passes.  A workgroup owns kWcTile consecutive nodes (small 3D cases: 16).  The nodes of
 // all their elements (the tile's nodes and a halo, listed once per mesh) are staged in LDS, and
-// kWcTileLanes (16) lanes per node walk the node's incident elements, finding each element's other nodes through
-// one 32-bit word of LDS slots (WcView::visit).  Reading the nodes from memory at every visit
+// kWcTileLanes lanes per node (2 in 2D, 4 in 3D; small 3D cases 16) walk the node's incident
+// elements, finding each element's other nodes through one 32-bit word of LDS slots
+// (WcView::visit).  Reading the nodes from memory at every visit
 // (d x 64 bytes, 24 visits per node in 3D) was bound by the rate at which the L1 looks up
 // scattered cache lines: the 3D momentum gather took the same time per visit on a mesh that
 // fits the L2 as on one 20 times larger, and halving its arithmetic gained 15 %.  A tile reads
