@@ -8,7 +8,7 @@
 //   w = omega B^-1 r                      (block-Jacobi pre-smoothing: at level 0 done by the
 //                                          BiCGSTAB kernel that forms r_0, on coarser levels by
 //                                          the restriction above)
-//   t = r - A w                           (k_amg_res; levels >= 1: k_amg_rr)
+//   t = r - A w                           (k_amg_res; levels >= 1: k_amg_rr or k_amg_res_nodes)
 //   r_{l+1} = P^T t                       (k_amg_restrict, gather over aggregate members; k_amg_rr)
 //   z_{l+1} = V-cycle(l+1)  /  A_c^-1 r_c (k_amg_tail, dense inverse on the coarsest)
 //   w' = w + alpha P z_{l+1}              (alpha > 1 over-corrects the piecewise-constant
@@ -41,6 +41,7 @@ __device__ __forceinline__ long long row_start_of(const int4& inf, int s, int D,
 }
 
 constexpr int kTailBlock = 1024;
+constexpr int kRrMembers = 64;  // members of an aggregate that k_amg_rr stages at a time
 
 }  // namespace
 
@@ -326,53 +327,80 @@ __global__ __launch_bounds__(kBlock) void k_amg_res(const AmgView<T>* __restrict
     PFEM_NF_MODE(res_rows, STREAM, V.A.nf, V.split, V, task, which);
 }
 
+// Residual of a level l >= 1 on its own, `lanes` lanes per node.
+template <typename T, int L>
+__device__ __forceinline__ void res_nodes(const AmgView<T>& V, const BlockTask& task) {
+    constexpr int NPB = kBlock / L;
+    const int lane = threadIdx.x % L, nf = V.A.nf;
+    for (long long i = (long long)task.block * NPB + threadIdx.x / L; i < V.A.N; i += (long long)task.nblocks * NPB) {
+        T y[kMaxNf];
+        node_spmv<L, true>(V.A, (const T*)V.w, i, lane, y);
+        if (lane < nf) V.t[i * nf + lane] = V.r[i * nf + lane] - pick(y, lane);
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_amg_res_nodes(const AmgView<T>* __restrict__ views,
+                                                          const BlockTask* __restrict__ tasks) {
+    const BlockTask task = tasks[blockIdx.x];
+    if (task.case_id < 0) return;
+    const AmgView<T>& V = views[task.case_id];
+    if (*V.done_flag) return;
+    if (V.lanes == 4) res_nodes<T, 4>(V, task);
+    else if (V.lanes == 8) res_nodes<T, 8>(V, task);
+    else res_nodes<T, 16>(V, task);
+}
+
+// Pre-smoothing of aggregate I on level l+1 (not the coarsest), field f: it is local to I.
+template <typename T>
+__device__ __forceinline__ void pre_smooth(const AmgView<T>& Vn, long long I, int f, int nf, int Nc,
+                                           const double (&sum)[kMaxNf]) {
+    T w = 0;
+#pragma unroll
+    for (int t = 0; t < kMaxNf; ++t)
+        if (t < nf) w = fma(Vn.binv[(long long)(f * nf + t) * Nc + I], (T)sum[t], w);
+    Vn.w[I * nf + f] = (T)Vn.omega * w;
+}
+
 // Residual and restriction of a level l >= 1 in one pass, a workgroup per aggregate: its lane
-// groups take the aggregate's members (every node of a coarse level has an aggregate), form
-// t = r - A w there and sum it per group in member order, then over the groups.  When level l+1
-// is not the coarsest its pre-smoothing follows, as in k_amg_restrict.
+// groups take the aggregate's members (every node of a coarse level has an aggregate) and form
+// t = r - A w there, then kRestrictLanes lanes per field sum it in k_amg_restrict's order.  The
+// launches of a large batch take k_amg_res_nodes and k_amg_restrict instead, which give the same bits.
 template <typename T, int L>
 __device__ __forceinline__ void rr_body(const AmgView<T>& V, const AmgView<T>& Vn, const BlockTask& task,
-                                        double (&red)[kWaves][kMaxNf]) {
-    const int lane = threadIdx.x % L, wl = threadIdx.x & 63, nf = V.A.nf, Nc = V.next_N;
-    const bool smooth = Vn.dense == nullptr;
+                                        T (&tl)[kRrMembers * kMaxNf], double (&red)[kMaxNf]) {
+    constexpr int R = kRestrictLanes;
+    static_assert(kRrMembers % R == 0 && R * kMaxNf <= 64, "a lane's members keep their order over the rounds");
+    const int lane = threadIdx.x % L, nf = V.A.nf, Nc = V.next_N, rl = threadIdx.x % R, rf = threadIdx.x / R;
     for (int I = task.block; I < Nc; I += task.nblocks) {
-        double acc[kMaxNf] = {0.0, 0.0, 0.0, 0.0};
-        for (int m = V.agg_ptr[I] + (int)threadIdx.x / L; m < V.agg_ptr[I + 1]; m += kBlock / L) {
-            const long long i = V.agg_nodes[m];
-            T y[kMaxNf];
-            node_spmv<L, true>(V.A, (const T*)V.w, i, lane, y);
-#pragma unroll
-            for (int s = 0; s < kMaxNf; ++s)
-                if (s < nf) {
-                    y[s] = V.r[i * nf + s] - y[s];
-                    acc[s] += (double)y[s];
+        const int m1 = V.agg_ptr[I + 1];
+        double acc = 0.0;
+        for (int m0 = V.agg_ptr[I]; m0 < m1; m0 += kRrMembers) {
+            const int cnt = min(kRrMembers, m1 - m0);
+            for (int m = threadIdx.x / L; m < cnt; m += kBlock / L) {
+                const long long i = V.agg_nodes[m0 + m];
+                T y[kMaxNf];
+                node_spmv<L, true>(V.A, (const T*)V.w, i, lane, y);
+                if (lane < nf) {
+                    const T t = V.r[i * nf + lane] - pick(y, lane);
+                    V.t[i * nf + lane] = t;
+                    tl[m * nf + lane] = t;
                 }
-            if (lane < nf) V.t[i * nf + lane] = pick(y, lane);
+            }
+            __syncthreads();
+            if (rf < nf)
+                for (int m = rl; m < cnt; m += R) acc += (double)tl[m * nf + rf];
+            __syncthreads();
         }
-#pragma unroll
-        for (int s = 0; s < kMaxNf; ++s) {
-#pragma unroll
-            for (int o = L; o < 64; o <<= 1) acc[s] += __shfl_xor(acc[s], o, 64);
-            if (wl == 0) red[threadIdx.x >> 6][s] = acc[s];
+        if (rf < nf) {
+            acc = group_sum<R>(acc);
+            if (rl == 0) red[rf] = acc;
         }
         __syncthreads();
         if ((int)threadIdx.x < nf) {
-            double sum[kMaxNf];
-#pragma unroll
-            for (int s = 0; s < kMaxNf; ++s) {
-                sum[s] = red[0][s];
-#pragma unroll
-                for (int w = 1; w < kWaves; ++w) sum[s] += red[w][s];
-            }
             const int f = threadIdx.x;
-            V.next_r[(long long)I * nf + f] = (T)pick(sum, f);
-            if (smooth) {
-                T w = 0;
-#pragma unroll
-                for (int t = 0; t < kMaxNf; ++t)
-                    if (t < nf) w += Vn.binv[(long long)(f * nf + t) * Nc + I] * (T)sum[t];
-                Vn.w[(long long)I * nf + f] = (T)Vn.omega * w;
-            }
+            V.next_r[(long long)I * nf + f] = (T)red[f];
+            if (Vn.dense == nullptr) pre_smooth(Vn, I, f, nf, Nc, red);
         }
         __syncthreads();
     }
@@ -386,16 +414,16 @@ __global__ __launch_bounds__(kBlock) void k_amg_rr(const AmgView<T>* __restrict_
     const AmgView<T>& V = views[task.case_id];
     if (*V.done_flag) return;
     const AmgView<T>& Vn = views[task.case_id + 1];  // level l+1 (views of a case are consecutive)
-    __shared__ double red[kWaves][kMaxNf];
-    if (V.lanes == 4) rr_body<T, 4>(V, Vn, task, red);
-    else if (V.lanes == 8) rr_body<T, 8>(V, Vn, task, red);
-    else rr_body<T, 16>(V, Vn, task, red);
+    __shared__ T tl[kRrMembers * kMaxNf];
+    __shared__ double red[kMaxNf];
+    if (V.lanes == 4) rr_body<T, 4>(V, Vn, task, tl, red);
+    else if (V.lanes == 8) rr_body<T, 8>(V, Vn, task, tl, red);
+    else rr_body<T, 16>(V, Vn, task, tl, red);
 }
 
-// Level 0: r_1(I, s) = sum over the members i of aggregate I of t(i, s) (full rows only);
+// r_{l+1}(I, s) = sum over the members i of aggregate I of t(i, s) (level 0: full rows only);
 // kRestrictLanes lanes per aggregate share its members (aggregates hold 5-30 nodes).  When
-// level 1 is not the coarsest, its pre-smoothing w_1(I) = omega B^-1(I) r_1(I) is local to I and
-// is applied here as well.
+// level l+1 is not the coarsest, its pre-smoothing is applied here as well.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_amg_restrict(const AmgView<T>* __restrict__ views,
                                                          const BlockTask* __restrict__ tasks) {
@@ -405,8 +433,6 @@ __global__ __launch_bounds__(kBlock) void k_amg_restrict(const AmgView<T>* __res
     const AmgView<T>& V = views[task.case_id];
     if (*V.done_flag) return;
     const AmgView<T>& Vn = views[task.case_id + 1];  // level l+1 (views of a case are consecutive)
-    const bool smooth = Vn.dense == nullptr;
-    const T om = (T)Vn.omega;
     const int nf = V.A.nf, D = nf - 1, Nc = V.next_N;
     const int lane = threadIdx.x % L;
     for (long long I = (long long)task.block * NPB + threadIdx.x / L; I < Nc; I += (long long)task.nblocks * NPB) {
@@ -423,13 +449,7 @@ __global__ __launch_bounds__(kBlock) void k_amg_restrict(const AmgView<T>* __res
             if (s < nf) acc[s] = group_sum<L>(acc[s]);
         if (lane < nf) {
             V.next_r[I * nf + lane] = (T)pick(acc, lane);
-            if (smooth) {
-                T w = 0;
-#pragma unroll
-                for (int t = 0; t < kMaxNf; ++t)
-                    if (t < nf) w += Vn.binv[(long long)(lane * nf + t) * Nc + I] * (T)acc[t];
-                Vn.w[I * nf + lane] = om * w;
-            }
+            if (Vn.dense == nullptr) pre_smooth(Vn, I, lane, nf, Nc, acc);
         }
     }
 }
@@ -596,6 +616,10 @@ void launch_amg_rr(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t 
     k_amg_rr<T><<<nt, kBlock, 0, s>>>(v, t);
 }
 template <typename T>
+void launch_amg_res_nodes(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t s) {
+    k_amg_res_nodes<T><<<nt, kBlock, 0, s>>>(v, t);
+}
+template <typename T>
 void launch_amg_tail(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t s) {
     k_amg_tail<T><<<nt, kTailBlock, 0, s>>>(v, t);
 }
@@ -616,6 +640,7 @@ void launch_amg_post(const AmgView<T>* v, const BlockTask* t, int nt, int which,
     template void launch_amg_res<T>(const AmgView<T>*, const BlockTask*, int, int, bool, hipStream_t); \
     template void launch_amg_restrict<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);   \
     template void launch_amg_rr<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);         \
+    template void launch_amg_res_nodes<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);  \
     template void launch_amg_tail<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);       \
     template void launch_amg_ap<T>(const AmgView<T>*, const BlockTask*, int, hipStream_t);         \
     template void launch_amg_post<T>(const AmgView<T>*, const BlockTask*, int, int, bool, hipStream_t);

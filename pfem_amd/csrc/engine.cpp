@@ -57,14 +57,30 @@ enum Tab : int {
     T_AMG = T_WCF + 2,  // multigrid tables: FP64 hierarchies, then FP32 ones (A_N each)
 };
 
+// Whether the V-cycle's last launch takes the level above the coarsest too.
+bool amg_tail(const pfem_case* c) {
+    const AmgHierarchy& H = c->amg;
+    const int last = H.levels - 1, nf = c->dim + 1;
+    return last >= 2 && H.lev[last - 1].N <= kAmgTailNodes && nf * nf * H.lev[last - 1].graph_nnz <= kAmgTailValues;
+}
+
+// Aggregates of a coarse level, over a tick's V-cycles, up to which its residual and restriction are
+// one launch with a workgroup per aggregate (2,048 run at once).  That launch saves ~4 us; beyond, its
+// workgroups of 5-30 short rows leave most lanes idle: the 512-request stream 208 steps/s with it at
+// every size, 229 up to 16,384, 231 up to 4,096 and 231 up to 1,024; 40 requests 105.4, 106.4,
+// 106.4 and 103.9 ms; without it 231 steps/s, 105.3 ms, and single cases 1-9 % slower (20k nodes
+// in 2D 15.2 / 13.9 ms, 60k in 3D 18.9 / 17.9).
+constexpr long long kRrAggregates = 2048;
+
 // Multigrid tables of one hierarchy type, relative to T_AMG + type * A_N: setup per level
 // (Galerkin, block Jacobi, A P), coarsest dense inverse; V-cycle per level (slices of the level-0
 // residual and of every level's post-smoothing, aggregates of the coarser levels' residual with
-// restriction, level 0's restriction), coarsest solve with the level above it.
+// restriction, restriction on its own, the coarser levels' residual on its own), coarsest solve with
+// the level above it.
 enum AmgTab : int {
     A_G = 0, A_B = A_G + kAmgMaxLevels, A_D = A_B + kAmgMaxLevels, A_AP = A_D + 1,
     A_VN = A_AP + kAmgMaxLevels, A_VS = A_VN + kAmgMaxLevels, A_VR = A_VS + kAmgMaxLevels,
-    A_VC = A_VR + kAmgMaxLevels, A_N = A_VC + 1
+    A_VE = A_VR + kAmgMaxLevels, A_VC = A_VE + kAmgMaxLevels, A_N = A_VC + 1
 };
 constexpr int T_NTAB = T_AMG + 2 * A_N;
 
@@ -1056,6 +1072,11 @@ void Engine::tick(std::vector<Req*>& done) {
     // ---- work tables ------------------------------------------------------------------
     std::vector<BlockTask> tab[T_NTAB];
     long long value_bytes = 0;            // matrices the tick's products read
+    long long vc_aggs[2][kAmgMaxLevels] = {};  // aggregates of each level >= 1 in the tick's V-cycles, by hierarchy type
+    for (Req* r : inflight_)
+        if ((r->ops & OP_K64_RUN) && pspg_like(r->c))
+            for (int l = 1; l + 1 < r->c->amg.levels - (amg_tail(r->c) ? 1 : 0); ++l)
+                vc_aggs[amg_fp32(r->c) ? 1 : 0][l] += r->c->amg.lev[l + 1].N;
     int wc_cap[2][2] = {{0, 0}, {0, 0}};  // most nodes a WC tile stages, by state type and dimension
     for (Req* r : inflight_) {
         pfem_case* c = r->c;
@@ -1104,15 +1125,18 @@ void Engine::tick(std::vector<Req*>& done) {
             }
             if (op & OP_K64_RUN) {
                 const int last = H.levels - 1;
-                const int nf = c->dim + 1;
-                const bool tail = last >= 2 && H.lev[last - 1].N <= kAmgTailNodes &&
-                                  nf * nf * H.lev[last - 1].graph_nnz <= kAmgTailValues;
+                const bool tail = amg_tail(c);
+                const long long* aggs = vc_aggs[amg_fp32(c) ? 1 : 0];
                 for (int l = 0; l < (tail ? last - 1 : last); ++l) {
                     const int Nl = l == 0 ? c->N : H.lev[l].N, nsl = (Nl + kEllSlice - 1) / kEllSlice;
                     const int nb = kry_blocks(nsl);
                     for (int b = 0; b < nb; ++b) A[A_VN + l].push_back(BlockTask{base + l, b, nb, 0});
-                    if (l > 0) append(A[A_VS + l], base + l, (long long)H.lev[l + 1].N * kBlock, kElemCap);
-                    else append(A[A_VR + l], base + l, (long long)H.lev[l + 1].N * kRestrictLanes, kElemCap);
+                    if (l > 0 && aggs[l] <= kRrAggregates) {
+                        append(A[A_VS + l], base + l, (long long)H.lev[l + 1].N * kBlock, kElemCap);
+                        continue;
+                    }
+                    if (l > 0) append(A[A_VE + l], base + l, (long long)Nl * H.lev[l].lanes, kElemCap);
+                    append(A[A_VR + l], base + l, (long long)H.lev[l + 1].N * kRestrictLanes, kElemCap);
                 }
                 A[A_VC].push_back(BlockTask{base + last, 0, 1, tail ? 1 : 0});
             }
@@ -1221,13 +1245,13 @@ void Engine::tick(std::vector<Req*>& done) {
     }
     // multigrid V-cycle of the cases that have a hierarchy: which = 0 (ph = M^-1 p) or 1 (sh = M^-1 s).
     // Level 0's residual and every level's post-smoothing walk ELL slices (table A_VN); residual
-    // and restriction of the coarser levels take a workgroup per aggregate (A_VS).
+    // and restriction of the coarser levels take a workgroup per aggregate (A_VS), in large batches
+    // a launch each (A_VE, A_VR).
     auto vcycle_type = [&](auto* v, int TA, int which) {
         for (int l = 0; l < kAmgMaxLevels; ++l) {
-            if (NT(TA + A_VR + l)) {
-                launch_amg_res(v, T(TA + A_VN + l), NT(TA + A_VN + l), which, stream, s);
-                launch_amg_restrict(v, T(TA + A_VR + l), NT(TA + A_VR + l), s);
-            }
+            if (l == 0 && NT(TA + A_VN)) launch_amg_res(v, T(TA + A_VN), NT(TA + A_VN), which, stream, s);
+            if (NT(TA + A_VE + l)) launch_amg_res_nodes(v, T(TA + A_VE + l), NT(TA + A_VE + l), s);
+            if (NT(TA + A_VR + l)) launch_amg_restrict(v, T(TA + A_VR + l), NT(TA + A_VR + l), s);
             if (NT(TA + A_VS + l)) launch_amg_rr(v, T(TA + A_VS + l), NT(TA + A_VS + l), s);
         }
         if (NT(TA + A_VC)) launch_amg_tail(v, T(TA + A_VC), NT(TA + A_VC), s);

@@ -36,6 +36,8 @@ void launch_amg_restrict(const AmgView<T>* v, const BlockTask* t, int nt, hipStr
 template <typename T>
 void launch_amg_rr(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t s);
 template <typename T>
+void launch_amg_res_nodes(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t s);
+template <typename T>
 void launch_amg_tail(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t s);
 template <typename T>
 void launch_amg_ap(const AmgView<T>* v, const BlockTask* t, int nt, hipStream_t s);
