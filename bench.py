@@ -464,15 +464,16 @@ def run_dambreak2d(ctx, steps=10, threads=1, with_cpu=True):
 # ------------------------------------------------------------------------------------------
 def wc_step_bytes(dim, nodes, elems, s_state):
     """Algorithmic bytes of one WC step with its computeNextDT (folded into the step's kernels):
-    connectivity read by the two element passes (continuity, momentum), the node state v, a
-    (dim each), p, rho read and written once, positions read and written once, and the FP64
-    accumulators (continuity mass and rhs, each node's smallest element size for the CFL,
-    momentum mass, dim force components) written and read once."""
-    conn = 2 * elems * (dim + 1) * 4
+    one 32-bit word per node-element incidence entry (the element's other nodes) read by the
+    continuity and the momentum pass, the node state v, a (dim each), p, rho read and written
+    once, positions read and written once, and what one pass leaves for the next written and
+    read once: each node's smallest element size (FP64, for the CFL), the half-step velocity and
+    the pressure before the continuity pass.  (The masses and forces stay in LDS.)"""
+    words = 2 * elems * (dim + 1) * 4
     state = 2 * nodes * (2 * dim + 2) * s_state
     pos = 2 * nodes * dim * 8
-    acc = 2 * nodes * (4 + dim) * 8
-    return conn + state + pos + acc
+    between = 2 * nodes * (8 + (dim + 1) * s_state)
+    return words + state + pos + between
 
 
 def run_wc3d(ctx, steps, warmup=3):
@@ -594,16 +595,19 @@ def spmv_fused_bytes(nodes, n, nnz, graph_nnz, vbytes=8):
     return nnz * vbytes + graph_nnz * 4 + (nodes + 1) * 4 + nodes * 16 + 3 * n * vbytes
 
 
+KRY_V = "k_kry_v<double, true>"  # the dam-break SpMV: FP64, non-temporal value loads
+
+
 def pmc_traffic(path=os.path.join(ROOT, "profiles", "spmv_kry_v_dambreak3d_262k_pmc_traffic.md")):
     """HBM bytes per launch of the dam-break SpMV from the committed rocprofv3 FETCH_SIZE /
     WRITE_SIZE passes (scaled by the counters' readings for a copy kernel of known size);
-    None when the summary is absent.  The counters need the profiler, so they cannot be read
+    None when the summary is absent or was measured on another kernel.  The counters need the profiler, so they cannot be read
     inside this process."""
     try:
         with open(path) as f:
-            for line in f:
-                if line.startswith("traffic_bytes_per_launch:"):
-                    return int(line.split(":")[1])
+            found = dict(line.strip().split(": ", 1) for line in f if line.startswith(("kernel: ", "traffic_bytes_per_launch: ")))
+        if found.get("kernel") == KRY_V:
+            return int(found["traffic_bytes_per_launch"])
     except OSError:
         pass
     return None
@@ -668,7 +672,7 @@ def run_dambreak3d(ctx, steps, warmup):
         elements_per_s=mesh.n_elems / t_asm if t_asm > 0 else None,
     )
     roof = {
-        "kernel": "k_kry_v<double> (BiCGSTAB SpMV v = A ph over the sliced ELL copy, fused (rh, v)), "
+        "kernel": f"{KRY_V} (BiCGSTAB SpMV v = A ph over the sliced ELL copy, fused (rh, v)), "
                   "3D dam break 262,701 nodes",
         "bound": "hbm",
         "achieved": achieved,

@@ -18,10 +18,12 @@
 // fits the L2 as on one 20 times larger, and halving its arithmetic gained 15 %.  A tile reads
 // ~7 node states per node instead of 72, mostly in runs.  On the 2.06M-node 3D tank (12M tets,
 // FP32 state) the six kernels of the record gathers (half 82, continuity element pass 280 and
-// gather 255, node pass 56, momentum gather 767, node pass 78 us) became half 34, continuity 379
-// and momentum 369 us; 100k nodes in FP64: 88 -> 60 us.  What bounds the tile passes now is FP64
-// issue (a visit is ~165 vector instructions in 3D, 200 us of the 369 at the full rate) and,
-// behind it, the latency of staging with four workgroups per CU.
+// gather 255, node pass 56, momentum gather 767, node pass 78 us) became half 33, continuity 379-432
+// and momentum 369-410 us (over GPUs); 100k nodes in FP64: 88 -> 60 us.  What bounds the tile passes
+// now, by the counters on that tank: with FP32 state vector issue (207 and 194 instructions per visit,
+// 63 % of the launch at a wave per 4 cycles and SIMD) and the LDS (half of it); with FP64 state the
+// LDS, three quarters of the launch, over half of it bank conflicts between lanes that read different
+// nodes; not HBM (1.46 GB per step in 0.87 ms).
 //
 // The P1 element quantities are the reference's Gauss-rule integrals in closed form:
 //   lump2(M(1))_i           = |e| / (d+1)
